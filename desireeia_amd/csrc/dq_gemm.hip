@@ -38,6 +38,7 @@
 
 #include "dq_common.h"
 #include "dq_f16.h"
+#include "dq_gemm_direct.h"
 
 namespace {
 
@@ -753,6 +754,7 @@ struct QuantDst {
     float* rscale;
     float* inv;
     int perm;        // 2 Q4_K fragment order, 1 Q6_K item order, 0 natural
+    int mp;          // 0: rows of lda halfs; else the direct kernel's slice order, mp = padded tokens
 };
 enum QuantSrcKind { Q_PLAIN = 0, Q_SILU = 1, Q_GELU = 2, Q_NORM = 3 };
 struct QuantSrc {
@@ -793,16 +795,21 @@ __device__ __forceinline__ void group_in(const QuantSrc& S, size_t row, int c, f
 // the block sum fs.
 __device__ __forceinline__ void store_group(const QuantDst& d, int lda, int n_tok, int t, int c, const h8& hv,
                                             float fs_scaled, bool sum_lane, bool ok) {
-    _Float16* o = d.out + (size_t)t * lda;
+    // where the 8 values of column `col` (a multiple of 8) of the row go
+    auto at = [&](int col) {
+        return reinterpret_cast<h8*>(
+            d.mp ? d.out + 8 * (((size_t)((col >> 8) * 8 + ((col >> 3) & 7)) * 4 + ((col >> 6) & 3)) * d.mp + t)
+                 : d.out + (size_t)t * lda + col);
+    };
     const int b = c / 4, q = c % 4;  // block, group in the block
     if (d.perm == 0) {
-        if (ok) *reinterpret_cast<h8*>(o + 8 * (size_t)c) = hv;
+        if (ok) *at(8 * c) = hv;
     } else if (d.perm == 1) {
         // Q6_K item order: position pos of the 256-block -> column s*256 +
         // (2n+k)*64 + qq*16 + e, pos = 128n + 32qq + 16k + e
         const int sb = b / 8, pos0 = 32 * (b % 8);
         const int n = pos0 / 128, qq = (pos0 % 128) / 32, k = q / 2;
-        if (ok) *reinterpret_cast<h8*>(o + sb * 256 + (2 * n + k) * 64 + qq * 16 + 8 * (q % 2)) = hv;
+        if (ok) *at(sb * 256 + (2 * n + k) * 64 + qq * 16 + 8 * (q % 2)) = hv;
     } else {
         // Q4_K fragment order: chunk (kk, hf) at column 16 kk + 8 hf of item i
         // holds elements e0..e0+3 (e0 = 16 hf + 4 kk) of the low block and of
@@ -827,7 +834,7 @@ __device__ __forceinline__ void store_group(const QuantDst& d, int lda, int n_to
         const int kk = 2 * (q % 2) + (hi ? 1 : 0), hf = q / 2;
         const h8 ch = {lo4[0], lo4[2], hi4[0], hi4[2], lo4[1], lo4[3], hi4[1], hi4[3]};
         if (!ok) return;
-        *reinterpret_cast<h8*>(o + 64 * (size_t)(b / 2) + 16 * kk + 8 * hf) = ch;
+        *at(64 * (b / 2) + 16 * kk + 8 * hf) = ch;
         if (sum_lane) d.minp[((size_t)(b / 8) * n_tok + t) * 8 + (b % 8)] = (_Float16)fs_scaled;
     }
 }
@@ -1008,6 +1015,16 @@ static size_t inv_off(int fmt, size_t cols, size_t n_tok) {
     return scale_off(fmt, cols, n_tok) + dq_align256(n_tok * 4);
 }
 
+// The same parts of the direct kernel's activation: tokens padded to 16, then
+// the block sums (part 0's end), s (1), 1/s (2); 3 is the total.
+static size_t direct_off(int fmt, size_t cols, size_t n_tok, int part) {
+    size_t off = dq_align256((n_tok + 15) / 16 * 16 * cols * 2);
+    if (part > 0) off += min_bytes(fmt, cols, n_tok);
+    if (part > 1) off += dq_align256(n_tok * 4);
+    if (part > 2) off += dq_align256(n_tok * 4);
+    return off;
+}
+
 extern "C" int dq_gemm_workspace_bytes(int fmt, size_t rows, size_t cols, size_t n_tok, size_t* bytes) {
     (void)rows;
     fmt &= ~DQ_FMT_GEMM_TILES;
@@ -1016,21 +1033,37 @@ extern "C" int dq_gemm_workspace_bytes(int fmt, size_t rows, size_t cols, size_t
         return DQ_ERR_NOT_SUPPORTED;
     if (cols % 256) return DQ_ERR_NOT_SUPPORTED;
     *bytes = inv_off(fmt, cols, n_tok) + dq_align256(n_tok * 4);
+    if (n_tok <= DQ_GEMM_DIRECT_TOK) {
+        const size_t d = direct_off(fmt, cols, n_tok, 3);
+        if (d > *bytes) *bytes = d;
+    }
     return DQ_OK;
 }
 
 static bool quant_fmt_ok(int fmt) {
     return fmt == DQ_FMT_Q4_K || fmt == DQ_FMT_Q6_K || fmt == DQ_FMT_Q8_0 || fmt == DQ_FMT_Q4_0;
 }
-static QuantDst quant_dst(int fmt, size_t cols, size_t n_tok, void* out) {
+static QuantDst quant_dst(int fmt, size_t cols, size_t n_tok, void* out, bool direct = false) {
     uint8_t* base = (uint8_t*)out;
     QuantDst d{};
     d.out = (_Float16*)base;
+    if (direct) {
+        d.mp = (int)((n_tok + 15) / 16 * 16);
+        d.minp = fmt == DQ_FMT_Q4_K ? (_Float16*)(base + direct_off(fmt, cols, n_tok, 0)) : nullptr;
+        d.rscale = (float*)(base + direct_off(fmt, cols, n_tok, 1));
+        d.inv = (float*)(base + direct_off(fmt, cols, n_tok, 2));
+        d.perm = fmt == DQ_FMT_Q6_K ? 1 : (fmt == DQ_FMT_Q4_K ? 2 : 0);
+        return d;
+    }
     d.minp = fmt == DQ_FMT_Q4_K ? (_Float16*)(base + min_off(cols, n_tok)) : nullptr;
     d.rscale = (float*)(base + scale_off(fmt, cols, n_tok));
     d.inv = (float*)(base + inv_off(fmt, cols, n_tok));
     d.perm = fmt == DQ_FMT_Q6_K ? 1 : (fmt == DQ_FMT_Q4_K ? 2 : 0);
     return d;
+}
+DqDirectAct dq_gemm_direct_act(int fmt, size_t cols, size_t n_tok, void* work) {
+    const QuantDst d = quant_dst(fmt, cols, n_tok, work, true);
+    return DqDirectAct{d.out, d.minp, d.inv};
 }
 // One workgroup per row of 64 (threads per row, up to 1024) times up to 8
 // groups of 8 columns per thread: rows of up to 65536 columns.
@@ -1054,12 +1087,12 @@ static int launch_quant_rows(const QuantSrc& S, size_t cols, size_t n_tok, const
 }
 
 int dq_quantize_act_f16_zero(int fmt, const float* d_x, size_t cols, size_t n_tok, void* d_out,
-                             const DqZeroSpans& z, void* stream, const float* d_gate, int act) {
+                             const DqZeroSpans& z, void* stream, const float* d_gate, int act, bool direct) {
     if (!quant_fmt_ok(fmt)) return DQ_ERR_NOT_SUPPORTED;
     if (cols % 256 || cols > QUANT_MAX_COLS || n_tok > (1u << 20)) return DQ_ERR_NOT_SUPPORTED;
     if (!d_x || !d_out) return DQ_ERR_INVALID_ARG;
     if (n_tok == 0) return DQ_OK;
-    const QuantDst d[2] = {quant_dst(fmt, cols, n_tok, d_out), QuantDst{}};
+    const QuantDst d[2] = {quant_dst(fmt, cols, n_tok, d_out, direct), QuantDst{}};
     QuantSrc S{};
     S.x = d_x;
     S.g = d_gate;
@@ -1072,7 +1105,7 @@ int dq_quantize_act_f16_zero(int fmt, const float* d_x, size_t cols, size_t n_to
 
 int dq_norm_quant_f16(const float* d_a, const float* d_b, float* d_h, const float* d_w, size_t cols, size_t n_tok,
                       float eps, float* d_y, int n_fmt, const int* fmts, void* const* outs, const DqZeroSpans& z,
-                      void* stream) {
+                      void* stream, bool direct) {
     if (n_fmt < 1 || n_fmt > 2 || !fmts || !outs || !d_a || !d_w) return DQ_ERR_INVALID_ARG;
     if (cols % 256 || cols > QUANT_MAX_COLS || n_tok > (1u << 20)) return DQ_ERR_NOT_SUPPORTED;
     if (n_tok == 0) return DQ_OK;
@@ -1080,7 +1113,7 @@ int dq_norm_quant_f16(const float* d_a, const float* d_b, float* d_h, const floa
     for (int k = 0; k < n_fmt; ++k) {
         if (!quant_fmt_ok(fmts[k])) return DQ_ERR_NOT_SUPPORTED;
         if (!outs[k]) return DQ_ERR_INVALID_ARG;
-        d[k] = quant_dst(fmts[k], cols, n_tok, outs[k]);
+        d[k] = quant_dst(fmts[k], cols, n_tok, outs[k], direct);
     }
     QuantSrc S{};
     S.x = d_a;
@@ -1333,6 +1366,13 @@ extern "C" int dq_gemm(int fmt_in, const void* d_w, size_t rows, size_t cols, co
     const int rc = dq_gemm_workspace_bytes(fmt, rows, cols, n_tok, &need);
     if (rc != DQ_OK) return rc;
     if (work_bytes < need || (need && !d_work)) return DQ_ERR_INVALID_ARG;
+    if (rows && n_tok && d_w && d_y && dq_gemm_direct_ok(fmt, rows, cols, n_tok)) {
+        const int rq = dq_quantize_act_f16_zero(fmt, d_x, cols, n_tok, d_work, DqZeroSpans{}, stream, nullptr, 0, true);
+        if (rq != DQ_OK) return rq;
+        const DqDirectJob j = {fmt, (fmt_in & DQ_FMT_GEMM_TILES) != 0, d_w, rows,
+                               dq_gemm_direct_act(fmt, cols, n_tok, d_work), d_y};
+        return dq_gemm_direct(&j, 1, cols, n_tok, (hipStream_t)stream);
+    }
     // the K-split plans add their partials into y: the quantizer clears it,
     // unless y overlaps x (the quantizer is still reading x), in which case
     // the GEMM launch clears y itself after the quantizer has finished

@@ -32,6 +32,7 @@
 #include <mutex>
 
 #include "dq_common.h"
+#include "dq_gemm_direct.h"
 #include "dq_f16.h"
 
 namespace {
@@ -881,6 +882,35 @@ int dq_layer_prefill(const dq_layer_t* L, const float* d_x, float* d_x_out, cons
     float* norm_h = nullptr;
     auto products = [&](const float* x, size_t cols, int n, const int* fmt, const void* const* wm, const size_t* rows,
                         float* const* y, const void* const* tm) -> int {
+        // few tokens: the direct kernel, all products of the input in one
+        // launch per format (Q4_K with Q6_K)
+        bool direct = true;
+        for (int j = 0; j < n; ++j) direct = direct && dq_gemm_direct_ok(fmt[j], rows[j], cols, T);
+        if (direct) {
+            bool made[3] = {false, false, false};
+            if (norm_w) {
+                int nf = 1, fq[2] = {fmt[0], 0};
+                for (int j = 1; j < n && nf < 2; ++j)
+                    if (cls(fmt[j]) != cls(fmt[0])) fq[nf++] = fmt[j];
+                void* outs[2] = {gw(fq[0]), nf > 1 ? gw(fq[1]) : nullptr};
+                for (int k = 0; k < nf; ++k) made[cls(fq[k])] = true;
+                bool third = false;
+                for (int j = 0; j < n; ++j) third |= !made[cls(fmt[j])];
+                DQP_TRY(dq_norm_quant_f16(norm_a, norm_b, norm_h, norm_w, cols, T, L->rms_eps,
+                                          third ? const_cast<float*>(x) : nullptr, nf, fq, outs, DqZeroSpans{}, s,
+                                          true));
+            }
+            DqDirectJob jobs[4];
+            for (int j = 0; j < n; ++j) {
+                if (!made[cls(fmt[j])])
+                    DQP_TRY(dq_quantize_act_f16_zero(fmt[j], x, cols, T, gw(fmt[j]), DqZeroSpans{}, s, glu_gate,
+                                                     glu_act, true));
+                made[cls(fmt[j])] = true;
+                jobs[j] = DqDirectJob{fmt[j], tm[j] != nullptr, tm[j] ? tm[j] : wm[j], rows[j],
+                                      dq_gemm_direct_act(fmt[j], cols, T, gw(fmt[j])), y[j]};
+            }
+            return dq_gemm_direct(jobs, n, cols, T, s);
+        }
         const int C = dq_gemm_cus();
         int budget[4] = {0, 0, 0, 0};
         SideStreams* ss = nullptr;
