@@ -133,6 +133,23 @@ __device__ __forceinline__ dq_u32x4 dq_ld16_stream(const void* p) {
 // __builtin_amdgcn_global_load_lds (direct global -> LDS DMA).
 #define DQ_LDS_PTR(p) reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(p))
 
+// A raw buffer over [p, p + bytes) (word 3: 32-bit data format) and the direct
+// load from it into LDS (lane i of the wave writes SIZE bytes at lds + SIZE i;
+// per-lane byte offset voff, wave-uniform soff). Out-of-range lanes load zero.
+// The buffer form keeps the compiler's wait counts exact: after a
+// global_load_lds, which is a FLAT instruction to it, every LDS read and
+// every plain load is waited for with a count of zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dq_buf(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+template <int SIZE>
+__device__ __forceinline__ void dq_buf_lds(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voff, uint32_t soff) {
+    static_assert(SIZE == 16 || SIZE == 4 || SIZE == 2, "bytes per lane");
+    if constexpr (SIZE == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, DQ_LDS_PTR(lds), 16, (int)voff, (int)soff, 0, 0);
+    if constexpr (SIZE == 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, DQ_LDS_PTR(lds), 4, (int)voff, (int)soff, 0, 0);
+    if constexpr (SIZE == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, DQ_LDS_PTR(lds), 2, (int)voff, (int)soff, 0, 0);
+}
+
 // DPP move of a float (gfx9 dpp_ctrl encodings; all rows and banks enabled).
 // Workgroup barrier for LDS rings filled by global_load_lds: waits for this
 // wave's LDS reads (lgkmcnt 0; gfx9 s_waitcnt encoding, vmcnt and expcnt at

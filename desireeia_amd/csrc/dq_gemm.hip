@@ -25,7 +25,7 @@
 // 128 tokens of its 64 rows over the kg-th share of the workgroup's K steps:
 // 4 x 2 v_mfma_f32_32x32x16_f16 tiles, so each weight fragment it turns into
 // fp16 feeds 4 MFMAs, and no other wave converts the same bytes. Each K group
-// has LDS rings filled by global_load_lds DMA: NS (2 or 3) activation stages
+// has LDS rings filled by direct global -> LDS DMA: NS (2 or 3) activation stages
 // of one K step (64 columns; XOR-swizzled 16-byte chunks, no bank conflicts
 // on fragment reads) and NB super-stages of SB packed weight items of the
 // group's rows (with the super-block header and, for Q4_K, the block sums
@@ -77,7 +77,7 @@ constexpr int kind_of() {
 // window: A (128-byte rows) the pairs (row parity, slot), SB 4 (64-byte rows)
 // the pairs (row % 4, slot) - swz = (row / 4) % 4 is distinct over the four
 // quads of either parity class - and SB 2 (32-byte rows) the pairs
-// (row % 8, slot). Every region is filled by global_load_lds (direct global -> LDS DMA: lane i of a
+// (row % 8, slot). Every region is filled by direct global -> LDS DMA (lane i of a
 // wave writes base + 16i, or base + 4i for the dword and sub-dword forms);
 // the plane DMA reads a row's SB*16 contiguous bytes with SB consecutive
 // lanes (whole cache-line pieces, not one 16-byte item of a different row
@@ -106,21 +106,6 @@ struct Ring {
 template <int SB>
 __device__ __forceinline__ int swz(int n) { return SB == 4 ? (n >> 2) & 3 : ((n >> 2) ^ (n >> 3)) & 1; }
 __device__ __forceinline__ int aswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-template <int SIZE>
-__device__ __forceinline__ void lds_dma(const void* g, uint8_t* lds_wave_base);
-template <>
-__device__ __forceinline__ void lds_dma<16>(const void* g, uint8_t* b) {
-    __builtin_amdgcn_global_load_lds(g, DQ_LDS_PTR(b), 16, 0, 0);
-}
-template <>
-__device__ __forceinline__ void lds_dma<4>(const void* g, uint8_t* b) {
-    __builtin_amdgcn_global_load_lds(g, DQ_LDS_PTR(b), 4, 0, 0);
-}
-template <>
-__device__ __forceinline__ void lds_dma<2>(const void* g, uint8_t* b) {
-    __builtin_amdgcn_global_load_lds(g, DQ_LDS_PTR(b), 2, 0, 0);
-}
 
 // s_waitcnt vmcnt(n), other counters untouched (gfx9 encoding: vmcnt in
 // bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
@@ -158,19 +143,6 @@ constexpr int b_loads() {
     return planes_of<KIND>() * SB + (KIND == B_Q4K ? 2 : KIND == B_Q40 ? 4 : KIND == B_Q6K ? 3 : 2);
 }
 
-template <int NWN, int KIND>
-__device__ __forceinline__ void issue_a(const GemmArgs& g, uint8_t* stage_base, int st, int wn, int lane) {
-    const int kcol = st * BK;
-#pragma unroll
-    for (int j = 0; j < a_loads<NWN>(); ++j) {
-        const int jj = j * NWN + wn;
-        const int slot = jj * 64 + lane;
-        const int r = slot >> 3, c = (slot & 7) ^ aswz(r);
-        const int m = min(g.m0 + r, g.M - 1);
-        lds_dma<16>(g.A + (size_t)m * g.lda + kcol + 8 * c, stage_base + jj * 64 * 16);
-    }
-}
-
 // Weight tiles (dq_gemm_tiles_pack, opt-in): for every 64-row slice of the
 // matrix and super-stage, the bytes one wave stages into its ring slot, in
 // the ring's own order (items already at their swizzled slots, the scales as
@@ -189,64 +161,102 @@ constexpr int tile_aux_bytes() { return KIND == B_Q4K ? 64 * 16 : KIND == B_Q6K 
 template <int KIND>
 constexpr int tile_slice_bytes() { return planes_of<KIND>() * tile_plane_bytes<KIND>() + tile_aux_bytes<KIND>(); }
 
-template <int NWN, int KIND, bool TL = false>
-__device__ __forceinline__ void issue_b(const GemmArgs& g, uint8_t* bb, int sb, int wn, int lane) {
-    using R = Ring<NWN, KIND>;
-    constexpr int SB = R::SB, BN = R::BN;
+// The buffers a workgroup's DMAs read and this lane's offsets in them, set up
+// once per tile (a step adds a wave-uniform offset): activations, block sums,
+// quant sub-planes (or the wave's tile slice) and scales.
+template <int NWN, int KIND>
+struct Src {
+    __amdgpu_buffer_rsrc_t a, m, q[planes_of<KIND>()], x, d;
+    uint32_t av[a_loads<NWN>()], mv, qv[sb_of<KIND>()], xv, dv;
+};
+
+template <int NWN, int KIND, bool TL>
+__device__ __forceinline__ void make_src(const GemmArgs& g, int wn, int lane, Src<NWN, KIND>& S) {
+    constexpr int SB = sb_of<KIND>();
+    const int m_rows = min(BM, g.M - g.m0), n_rows = min(64 * NWN, g.N - g.n0);
+    S.a = dq_buf(g.A + (size_t)g.m0 * g.lda, (uint32_t)m_rows * g.lda * 2);
+#pragma unroll
+    for (int j = 0; j < a_loads<NWN>(); ++j) {
+        const int slot = (j * NWN + wn) * 64 + lane;
+        const int r = slot >> 3, c = (slot & 7) ^ aswz(r);
+        S.av[j] = (uint32_t)min(r, m_rows - 1) * (uint32_t)g.lda * 2 + 16 * c;
+    }
+    if constexpr (KIND == B_Q4K) {
+        S.m = dq_buf(g.minp + (size_t)g.m0 * 8, (uint32_t)((size_t)(g.K / 256 - 1) * g.M + m_rows) * 16);
+        S.mv = (uint32_t)min((wn & 1) * 64 + lane, m_rows - 1) * 16;
+    }
     if constexpr (TL) {
-        constexpr int PL = tile_plane_bytes<KIND>();
-        const uint8_t* src = g.w + ((size_t)(g.n0 / 64 + wn) * g.n_stages + sb) * tile_slice_bytes<KIND>();
-#pragma unroll
-        for (int p = 0; p < planes_of<KIND>(); ++p)
-#pragma unroll
-            for (int k = 0; k < SB; ++k)
-                lds_dma<16>(src + p * PL + (64 * k + lane) * 16, bb + p * R::PLANE + (64 * wn * SB + 64 * k) * 16);
-        const uint8_t* aux = src + planes_of<KIND>() * PL;
-        if constexpr (KIND == B_Q4K) {
-            lds_dma<16>(aux + lane * 16, bb + R::AUX + 64 * wn * 16);
-            const int blk = wn & 1, m = min(g.m0 + blk * 64 + lane, g.M - 1);
-            lds_dma<16>(g.minp + ((size_t)sb * g.M + m) * 8, bb + R::MIN + blk * 64 * 16);
-        } else {
-            constexpr int NA = KIND == B_Q6K ? 3 : SB;  // 4-byte aux slots per row
-#pragma unroll
-            for (int c = 0; c < NA; ++c) lds_dma<4>(aux + c * 256 + lane * 4, bb + R::AUX + c * BN * 4 + 64 * wn * 4);
-        }
+        S.q[0] = dq_buf(g.w + (size_t)(g.n0 / 64 + wn) * g.n_stages * tile_slice_bytes<KIND>(),
+                        (uint32_t)g.n_stages * tile_slice_bytes<KIND>());
         return;
     }
-    const int item0 = SB * sb;
-    // planes: instruction k covers own rows 64 SB^-1 ... : slot s = 64k + lane
 #pragma unroll
-    for (int p = 0; p < planes_of<KIND>(); ++p) {
+    for (int p = 0; p < planes_of<KIND>(); ++p)
+        S.q[p] = dq_buf(g.w + g.L.q_off + p * g.L.p_stride + (size_t)g.n0 * g.L.q_row, (uint32_t)(n_rows * g.L.q_row));
 #pragma unroll
-        for (int k = 0; k < SB; ++k) {
-            const int s = 64 * k + lane;
-            const int n = 64 * wn + s / SB;                 // row in the tile
-            const int t = (s % SB) ^ swz<SB>(n);            // the item this LDS slot holds
-            const size_t r = (size_t)min(g.n0 + n, g.N - 1);
-            const uint8_t* src = g.w + g.L.q_off + p * g.L.p_stride + r * g.L.q_row + 16 * (size_t)(item0 + t);
-            lds_dma<16>(src, bb + p * R::PLANE + (64 * wn * SB + 64 * k) * 16);
-        }
+    for (int k = 0; k < SB; ++k) {
+        const int s = 64 * k + lane;
+        const int n = 64 * wn + s / SB;       // row in the tile
+        const int t = (s % SB) ^ swz<SB>(n);  // the item this LDS slot holds
+        S.qv[k] = (uint32_t)min(n, n_rows - 1) * (uint32_t)g.L.q_row + 16 * t;
     }
-    const int n = 64 * wn + lane;
-    const size_t r = (size_t)min(g.n0 + n, g.N - 1);
+    const uint32_t n = (uint32_t)min(64 * wn + lane, n_rows - 1);
+    if constexpr (KIND == B_Q4K || KIND == B_Q6K) {
+        S.x = dq_buf(g.w + g.L.s_off + (size_t)g.n0 * g.L.s_row, (uint32_t)(n_rows * g.L.s_row));
+        S.xv = n * (uint32_t)g.L.s_row;
+    }
+    if constexpr (KIND != B_Q4K) {
+        S.d = dq_buf(g.w + g.L.d_off + (size_t)g.n0 * g.L.d_row, (uint32_t)(n_rows * g.L.d_row));
+        S.dv = n * (uint32_t)g.L.d_row;
+    }
+}
+
+template <int NWN, int KIND>
+__device__ __forceinline__ void issue_a(const Src<NWN, KIND>& S, uint8_t* stage_base, int st, int wn) {
+#pragma unroll
+    for (int j = 0; j < a_loads<NWN>(); ++j)
+        dq_buf_lds<16>(S.a, stage_base + (j * NWN + wn) * 64 * 16, S.av[j], (uint32_t)(st * BK * 2));
+}
+
+// DMA instruction i (0 .. b_loads() - 1) of B super-stage sb: the planes' SB
+// instructions each, then the scales, then (Q4_K) the block sums.
+template <int NWN, int KIND, bool TL>
+__device__ __forceinline__ void issue_b1(const GemmArgs& g, const Src<NWN, KIND>& S, uint8_t* bb, int sb, int wn,
+                                         int lane, int i) {
+    using R = Ring<NWN, KIND>;
+    constexpr int SB = R::SB, BN = R::BN, NP = planes_of<KIND>(), PL = tile_plane_bytes<KIND>();
     uint8_t* aux = bb + R::AUX;
-    if constexpr (KIND == B_Q4K) {
-        lds_dma<16>(g.w + g.L.s_off + r * g.L.s_row + 16 * (size_t)sb, aux + 64 * wn * 16);
-        const int blk = wn & 1, m = min(g.m0 + blk * 64 + lane, g.M - 1);
-        lds_dma<16>(g.minp + ((size_t)sb * g.M + m) * 8, bb + R::MIN + blk * 64 * 16);
-    } else if constexpr (KIND == B_Q6K) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-            lds_dma<4>(g.w + g.L.s_off + r * g.L.s_row + 4 * (size_t)(item0 + c), aux + c * BN * 4 + 64 * wn * 4);
-        // a sub-dword LDS DMA still advances 4 bytes per lane: d sits in the
-        // low half of a dword slot
-        lds_dma<2>(g.w + g.L.d_off + r * g.L.d_row + 2 * (size_t)(item0 >> 2), aux + 2 * BN * 4 + 64 * wn * 4);
-    } else {
-        constexpr int ND = KIND == B_Q80 ? 2 : 4;  // one dword (two fp16 block scales) per item
-#pragma unroll
-        for (int c = 0; c < ND; ++c)
-            lds_dma<4>(g.w + g.L.d_off + r * g.L.d_row + 4 * (size_t)(item0 + c), aux + c * BN * 4 + 64 * wn * 4);
+    const uint32_t run = TL ? (uint32_t)sb * tile_slice_bytes<KIND>() : 0u, item0 = SB * sb;
+    if (i < NP * SB) {  // instruction k of a plane covers slots 64k + lane of the wave's 64 rows
+        const int p = i / SB, k = i % SB;
+        uint8_t* dst = bb + p * R::PLANE + (64 * wn * SB + 64 * k) * 16;
+        if constexpr (TL) dq_buf_lds<16>(S.q[0], dst, lane * 16, run + p * PL + 1024 * k);
+        else dq_buf_lds<16>(S.q[p], dst, S.qv[k], 16 * item0);
+        return;
     }
+    const int c = i - NP * SB;
+    const uint32_t ax = run + NP * PL;
+    if constexpr (KIND == B_Q4K) {
+        if (c == 1) {
+            dq_buf_lds<16>(S.m, bb + R::MIN + (wn & 1) * 64 * 16, S.mv, (uint32_t)(sb * g.M * 16));
+        } else {
+            if constexpr (TL) dq_buf_lds<16>(S.q[0], aux + 64 * wn * 16, lane * 16, ax);
+            else dq_buf_lds<16>(S.x, aux + 64 * wn * 16, S.xv, 16 * (uint32_t)sb);
+        }
+    } else {  // 4-byte slots: Q6_K the two items' scales, then d in the low half (a
+              // sub-dword LDS DMA still advances 4 bytes per lane); Q8_0, Q4_0 an item's two d
+        uint8_t* dst = aux + c * BN * 4 + 64 * wn * 4;
+        if constexpr (TL) dq_buf_lds<4>(S.q[0], dst, lane * 4, ax + c * 256);
+        else if (KIND == B_Q6K && c == 2) dq_buf_lds<2>(S.d, dst, S.dv, 2 * (item0 >> 2));
+        else if constexpr (KIND == B_Q6K) dq_buf_lds<4>(S.x, dst, S.xv, 4 * (item0 + c));
+        else dq_buf_lds<4>(S.d, dst, S.dv, 4 * (item0 + c));
+    }
+}
+template <int NWN, int KIND, bool TL>
+__device__ __forceinline__ void issue_b(const GemmArgs& g, const Src<NWN, KIND>& S, uint8_t* bb, int sb, int wn,
+                                        int lane) {
+#pragma unroll
+    for (int i = 0; i < b_loads<KIND>(); ++i) issue_b1<NWN, KIND, TL>(g, S, bb, sb, wn, lane, i);
 }
 
 __device__ __forceinline__ const h8& lds_h8(const uint8_t* p) { return *reinterpret_cast<const h8*>(p); }
@@ -349,57 +359,59 @@ __device__ __forceinline__ void b_scales(const BRaw& r, int G, BScale& S) {
     b_scales_j<KIND>(r, G, S, 1);
 }
 
-template <int KIND, int KK>
-__device__ __forceinline__ h8 b_frag_j(const BRaw& r, const BScale& S, int j) {
-    {
-        uint32_t t[4];
-        if constexpr (KIND == B_Q4K) {
-            // Slice KK: word KK of sub-plane h (lane half h holds all 16 bytes
-            // of sub-plane h). From the dword's bytes B0..B3, a nibble ORed into mantissa bits
-            // 7:4 under the exponent of 64 (0x5400) is the fp16 64 + q exactly,
-            // two per v_and_or; fma(64 + q, a, -64a) = q*a rounded once (as
-            // (q)*a would be). Fragment order (the activation tile is permuted
-            // to match, dq_quantize_act_f16): lo B0, lo B2, hi B0, hi B2, lo B1,
-            // lo B3, hi B1, hi B3; lo = sub-block 2G (scale a0), hi = 2G+1 (a1).
-            const dq_u32x2 src = KK < 2 ? r.q0[j] : r.q1[j];
-            const uint32_t w = (KK & 1) ? src.y : src.x;
-            // the exponent pattern comes from a register (S.magic): with both
-            // operands literal the compiler splits each v_and_or into two
-            const uint32_t e0 = ((w << 4) & 0x00F000F0u) | S.magic;
-            const uint32_t e1 = (w & 0x00F000F0u) | S.magic;
-            const uint32_t e2 = ((w >> 4) & 0x00F000F0u) | S.magic;
-            const uint32_t e3 = ((w >> 8) & 0x00F000F0u) | S.magic;
-            t[0] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, e0), S.s[j][0], S.s[j][2]));
-            t[1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, e1), S.s[j][1], S.s[j][3]));
-            t[2] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, e2), S.s[j][0], S.s[j][2]));
-            t[3] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, e3), S.s[j][1], S.s[j][3]));
-        } else if constexpr (KIND == B_Q80) {
-            // slice KK = sub-plane KK, bytes 8h..8h+7: q ^ 0x80 = q + 128 under
-            // the exponent of 1024, minus 1152 = q exactly, times d (one rounding)
-            const h2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-            const dq_u32x2 src = KK == 0 ? r.q0[j] : KK == 1 ? r.q1[j] : KK == 2 ? r.q2[j] : r.q3[j];
-            bytes_to_h2(src.x ^ 0x80808080u, bias, S.s[j][KK], &t[0]);
-            bytes_to_h2(src.y ^ 0x80808080u, bias, S.s[j][KK], &t[2]);
-        } else if constexpr (KIND == B_Q40) {
-            // slices 0, 1: sub-plane 0 (block 2i) low, high nibbles; 2, 3: sub-plane 1;
-            // the nibble q under the exponent of 1024, minus 1032 = q - 8, times d
-            const h2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-            const dq_u32x2 src = KK < 2 ? r.q0[j] : r.q1[j];
-            const int sh = (KK & 1) ? 4 : 0;
-            bytes_to_h2((src.x >> sh) & 0x0F0F0F0Fu, bias, S.s[j][KK], &t[0]);
-            bytes_to_h2((src.y >> sh) & 0x0F0F0F0Fu, bias, S.s[j][KK], &t[2]);
-        } else {
-            const h2 bias = {(_Float16)1056.0f, (_Float16)1056.0f};  // 1024 + 32
-            const dq_u32x2 lo = (KK & 1) ? r.q1[j] : r.q0[j];
-#pragma unroll
-            for (int wd = 0; wd < 2; ++wd) {
-                const uint32_t l4 = KK < 2 ? (lo[wd] & 0x0F0F0F0Fu) : ((lo[wd] >> 4) & 0x0F0F0F0Fu);
-                const uint32_t v6 = l4 | (((r.q2[j][wd] >> (2 * KK)) & 0x03030303u) << 4);
-                bytes_to_h2(v6, bias, S.s[j][KK], &t[2 * wd]);
+// Word K (two weights) of the 4-word fragment of slice KK, row block j; v
+// carries a source dword from an even word to the next odd one.
+template <int KIND, int KK, int K>
+__device__ __forceinline__ uint32_t b_word(const BRaw& r, const BScale& S, int j, uint32_t& v) {
+    if constexpr (KIND == B_Q4K) {
+        // Slice KK: word KK of sub-plane h (lane half h holds all 16 bytes
+        // of sub-plane h). From the dword's bytes B0..B3, a nibble ORed into mantissa bits
+        // 7:4 under the exponent of 64 (0x5400) is the fp16 64 + q exactly,
+        // two per v_and_or; fma(64 + q, a, -64a) = q*a rounded once (as
+        // (q)*a would be). Fragment order (the activation tile is permuted
+        // to match, dq_quantize_act_f16): lo B0, lo B2, hi B0, hi B2, lo B1,
+        // lo B3, hi B1, hi B3; lo = sub-block 2G (scale a0), hi = 2G+1 (a1).
+        // The exponent pattern comes from a register (S.magic): with both
+        // operands literal the compiler splits each v_and_or into two.
+        const dq_u32x2 src = KK < 2 ? r.q0[j] : r.q1[j];
+        const uint32_t w = (KK & 1) ? src.y : src.x;
+        const uint32_t sh = K == 0 ? w << 4 : K == 1 ? w : K == 2 ? w >> 4 : w >> 8;
+        const uint32_t e = (sh & 0x00F000F0u) | S.magic;
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, e), S.s[j][K & 1],
+                                                                      S.s[j][2 + (K & 1)]));
+    } else {
+        // Q8_0: slice KK = sub-plane KK, bytes 8h..8h+7: q ^ 0x80 = q + 128 under
+        // the exponent of 1024, minus 1152 = q exactly, times d (one rounding).
+        // Q4_0: slices 0, 1 = sub-plane 0 (block 2i) low, high nibbles; 2, 3
+        // sub-plane 1; the nibble q under the exponent of 1024, minus 1032.
+        // Q6_K: the 6-bit q under it, minus 1056.
+        constexpr int W = K / 2;
+        const _Float16 b = KIND == B_Q80 ? (_Float16)1152.0f : KIND == B_Q40 ? (_Float16)1032.0f : (_Float16)1056.0f;
+        if constexpr (K % 2 == 0) {
+            if constexpr (KIND == B_Q80) {
+                const dq_u32x2 src = KK == 0 ? r.q0[j] : KK == 1 ? r.q1[j] : KK == 2 ? r.q2[j] : r.q3[j];
+                v = src[W] ^ 0x80808080u;
+            } else if constexpr (KIND == B_Q40) {
+                const dq_u32x2 src = KK < 2 ? r.q0[j] : r.q1[j];
+                v = (src[W] >> ((KK & 1) ? 4 : 0)) & 0x0F0F0F0Fu;
+            } else {
+                const dq_u32x2 lo = (KK & 1) ? r.q1[j] : r.q0[j];
+                const uint32_t l4 = KK < 2 ? (lo[W] & 0x0F0F0F0Fu) : ((lo[W] >> 4) & 0x0F0F0F0Fu);
+                v = l4 | (((r.q2[j][W] >> (2 * KK)) & 0x03030303u) << 4);
             }
         }
-        return __builtin_bit_cast(h8, dq_u32x4{t[0], t[1], t[2], t[3]});
+        const h2 p = (magic_pair(v, K % 2 == 0 ? 0x04010400u : 0x04030402u) - h2{b, b}) * S.s[j][KK];
+        return __builtin_bit_cast(uint32_t, p);
     }
+}
+template <int KIND, int KK>
+__device__ __forceinline__ h8 b_frag_j(const BRaw& r, const BScale& S, int j) {
+    uint32_t v = 0, t[4];
+    t[0] = b_word<KIND, KK, 0>(r, S, j, v);
+    t[1] = b_word<KIND, KK, 1>(r, S, j, v);
+    t[2] = b_word<KIND, KK, 2>(r, S, j, v);
+    t[3] = b_word<KIND, KK, 3>(r, S, j, v);
+    return __builtin_bit_cast(h8, dq_u32x4{t[0], t[1], t[2], t[3]});
 }
 
 template <int KIND, int KK>
@@ -430,22 +442,38 @@ struct Pre {
     h8 bm[2];
 };
 
-// s_waitcnt vmcnt at the middle of a step of phase T: the A stage of the next
-// step must have landed (and, at the last phase, this wave's part of the next
-// B super-stage). DMAs are issued in the middle of each step - A(st + NS),
-// then at phase 0 the B super-stage NB-1 ahead - so the count of DMA
-// instructions issued after the needed one depends only on the phase.
+// DMA instructions issued in the last slice of a step of phase T: the
+// activation stage NS steps ahead, and half of the B super-stage NB - 1 ahead
+// in each of the phases 0 and 1.
+template <int KIND, int T>
+constexpr int b_first() { return T == 0 ? 0 : b_loads<KIND>() / 2; }
+template <int KIND, int T>
+constexpr int b_count() { return T == 0 ? b_loads<KIND>() / 2 : T == 1 ? b_loads<KIND>() - b_loads<KIND>() / 2 : 0; }
+template <int KIND>
+constexpr int b_count_at(int t) { return t == 0 ? b_count<KIND, 0>() : t == 1 ? b_count<KIND, 1>() : 0; }
+
+// s_waitcnt vmcnt before the last slice of a step of phase T, for the A stage
+// of the next step (issued NS - 1 steps back, before that step's B part): the
+// DMAs issued after it may stay in flight.
 template <int NWN, int KIND, int NS, int T>
 constexpr int mid_wait() {
-    constexpr int SB = sb_of<KIND>(), PA = a_loads<NWN>(), PB = b_loads<KIND>();
-    // A(st+1) was issued NS-1 steps back; B issues in between at phase 0
+    constexpr int SB = sb_of<KIND>(), PA = a_loads<NWN>();
     int w = 0;
     for (int back = NS - 1; back >= 1; --back) {
-        // issues of step st - back, after A(st+1) itself (which is issued by step st+1-NS)
         const int ph = ((T - back) % SB + SB) % SB;
-        if (back < NS - 1) w += PA;          // A issued by a later step
-        if (ph == 0) w += PB;                 // that step's B issue (after its A)
+        if (back < NS - 1) w += PA;
+        w += b_count_at<KIND>(ph);
     }
+    return w;
+}
+// s_waitcnt vmcnt at the start of a super-stage's last step, for this wave's
+// part of the next B super-stage (its second half issued in phase 1, NB - 1
+// super-stages earlier): the DMAs issued after it may stay in flight.
+template <int NWN, int KIND>
+constexpr int b_wait() {
+    constexpr int SB = sb_of<KIND>(), NB = SB == 4 ? 2 : 3, PA = a_loads<NWN>();
+    int w = 0;
+    for (int t = -(NB - 2) * SB + 2; t < SB - 1; ++t) w += PA + b_count_at<KIND>((t + 2 * SB) % SB);
     return w;
 }
 
@@ -454,122 +482,140 @@ __device__ __forceinline__ h8 a_frag(const uint8_t* base, int kk, int i, int lan
     return lds_h8(base + (r * 8 + ((2 * kk + (lane >> 5)) ^ aswz(r))) * 16);
 }
 
-// MFMA q of a slice (32x32 block i = q/2 of the tokens, j = q%2 of the rows),
-// and the pin that keeps the companion work written after it in place: a
-// wave issues in order and an MFMA waits for the matrix pipe, so the LDS
-// reads and conversions of the next slice are placed one or two per MFMA
-// rather than in runs the scheduler would build (a run of MFMAs holds back
-// every instruction behind it).
+// Slot Q of a slice: MFMA Q (32x32 block i = Q/2 of the tokens, j = Q%2 of
+// the rows) and after it a piece of the companion work, pinned in place. A
+// wave alone on its SIMD issues in order: after an MFMA its next VALU
+// instruction waits 16 cycles, and the next MFMA 32 (a 32x32x16 takes 32), so
+// up to four VALU instructions per slot cost nothing and more add 4 cycles
+// each; LDS reads move 64 bytes per cycle for the whole CU (16 cycles per
+// 1 KB fragment), which the four activation fragments of a slice and wave
+// fill. So the conversion of the next slice's weights goes one word (2-4
+// instructions) to a slot, and the LDS reads and DMAs one to a slot, instead
+// of in runs.
 #define DQ_MF(AF, BF, Q) \
     acc[(Q) >> 1][(Q)&1] = __builtin_amdgcn_mfma_f32_32x32x16_f16((AF)[(Q) >> 1], (BF)[(Q)&1], acc[(Q) >> 1][(Q)&1], 0, 0, 0)
 #define DQ_PIN() __builtin_amdgcn_sched_barrier(0)
+// slot Q of slice SL < 3: slice SL + 1's fragments, and further work W
+#define DQ_SLOT(AF, BF, SL, Q, W)                                                       \
+    DQ_MF(AF, BF, Q);                                                                   \
+    if constexpr ((Q) % 2 == 0) afn[(Q) / 2] = a_frag(abase, SL + 1, (Q) / 2, lane);   \
+    tw[(Q) / 4][(Q) % 4] = b_word<KIND, SL + 1, (Q) % 4>(P.raw, P.S, (Q) / 4, v);      \
+    W;                                                                                  \
+    DQ_PIN()
+#define DQ_TAKE()                                                                                    \
+    _Pragma("unroll") for (int i = 0; i < 4; ++i) afc[i] = afn[i];                                   \
+    _Pragma("unroll") for (int j = 0; j < 2; ++j)                                                    \
+        bfc[j] = __builtin_bit_cast(h8, dq_u32x4{tw[j][0], tw[j][1], tw[j][2], tw[j][3]})
 
 // One K step st (phase T of super-stage sb) of a wave whose registers P hold
-// the step's slice-0 fragments. Slices 0-2: each MFMA is followed by a piece
-// of the next slice's work (its four activation fragments, LDS; its weight
-// fragments, VALU) and, within a super-stage, of the next step's B side (this
-// wave's own rows: raw bytes, scales, slice-0 fragments). Then, once every A
-// read of the step is issued: the wait for the next step's stage, the
-// workgroup barrier (this stage free, the next one visible), the DMAs into
-// the freed stage (and at phase 0 the B super-stage NB-1 ahead), and slice
-// 3 with the next step's slice-0 activation fragments; at the last phase the
-// next super-stage's B side (landed by the wait), overlapped with the Q4_K
-// min-term slice. Q4_K builds the min-term weight fragments in phase 1.
+// the step's slice-0 fragments. Beside the MFMAs of slices 0-2: the next
+// slice's activation fragments (LDS) and weight fragments, the raw bytes and
+// scales of the next step's weights (this wave's own rows, no barrier: at the
+// super-stage's last step the next one's, waited for at the step's start).
+// Then, once every A read of the step is issued: the wait for the next step's
+// stage, the workgroup barrier (this stage free, the next one visible), and
+// slice 3 with the next step's slice-0 fragments and the DMAs into the freed
+// stage. Q4_K: the min-term weight fragments are built in phase 1, their
+// slice runs at the end of the super-block's last step.
 template <int NWN, int KIND, int NS, int T, bool TL>
-__device__ __forceinline__ void gemm_step(const GemmArgs& g, uint8_t* aring, uint8_t* bring, int& astage, int sb,
-                                          int a_next, int b_next, Pre& P, f16v (&acc)[4][2], int wn, int lane) {
+__device__ __forceinline__ void gemm_step(const GemmArgs& g, const Src<NWN, KIND>& src, uint8_t* aring, uint8_t* bring,
+                                          int& astage, int sb, int a_next, int b_next, Pre& P, f16v (&acc)[4][2],
+                                          int wn, int lane) {
     using R = Ring<NWN, KIND>;
-    constexpr int SB = R::SB, NB = R::NB;
+    constexpr int SB = R::SB, NB = R::NB, PA = a_loads<NWN>(), NBI = b_count<KIND, T>();
     constexpr bool LAST = T + 1 == SB;
     constexpr int T1 = LAST ? 0 : T + 1;
     constexpr bool MINT = KIND == B_Q4K && T == 3;  // min-term slice
+    constexpr bool MINB = KIND == B_Q4K && T == 1;  // its weight fragments
     const uint8_t* abase = aring + astage * R::A_STAGE;
     const uint8_t* bbase = bring + (sb % NB) * R::B_STAGE;
     const int next_stage = astage + 1 == NS ? 0 : astage + 1;
     const uint8_t* anext = aring + next_stage * R::A_STAGE;
-    const uint8_t* bnext = bring + ((sb + 1) % NB) * R::B_STAGE;
-    h8 af1[4], af2[4], af3[4], bf1[2], bf2[2], bf3[2], bn[2], am[4];
+    const uint8_t* braw = LAST ? bring + ((sb + 1) % NB) * R::B_STAGE : bbase;
+    uint8_t* bdst = bring + (b_next % NB) * R::B_STAGE;
+    h8 afn[4], afc[4], bfc[2], am[4];
+    uint32_t tw[2][4], v = 0;
     BRaw rn;
     BScale sn;
     sn.magic = P.S.magic;
-    // slice 0
-    DQ_MF(P.af, P.bf, 0); af1[0] = a_frag(abase, 1, 0, lane); DQ_PIN();
-    DQ_MF(P.af, P.bf, 1); af1[1] = a_frag(abase, 1, 1, lane); DQ_PIN();
-    DQ_MF(P.af, P.bf, 2); af1[2] = a_frag(abase, 1, 2, lane); DQ_PIN();
-    DQ_MF(P.af, P.bf, 3); af1[3] = a_frag(abase, 1, 3, lane); DQ_PIN();
-    DQ_MF(P.af, P.bf, 4); bf1[0] = b_frag_j<KIND, 1>(P.raw, P.S, 0); DQ_PIN();
-    DQ_MF(P.af, P.bf, 5); if constexpr (!LAST) b_raw_j<NWN, KIND>(bbase, T1, wn, lane, rn, 0); DQ_PIN();
-    DQ_MF(P.af, P.bf, 6); bf1[1] = b_frag_j<KIND, 1>(P.raw, P.S, 1); DQ_PIN();
-    DQ_MF(P.af, P.bf, 7); if constexpr (!LAST) b_raw_j<NWN, KIND>(bbase, T1, wn, lane, rn, 1); DQ_PIN();
-    // slice 1
-    DQ_MF(af1, bf1, 0); af2[0] = a_frag(abase, 2, 0, lane); DQ_PIN();
-    DQ_MF(af1, bf1, 1); if constexpr (KIND == B_Q4K && T == 1) P.bm[0] = q4k_neg_mins(P.raw.hd[0], true); DQ_PIN();
-    DQ_MF(af1, bf1, 2); af2[1] = a_frag(abase, 2, 1, lane); af2[2] = a_frag(abase, 2, 2, lane); DQ_PIN();
-    DQ_MF(af1, bf1, 3); if constexpr (KIND == B_Q4K && T == 1) P.bm[1] = q4k_neg_mins(P.raw.hd[1], true); DQ_PIN();
-    DQ_MF(af1, bf1, 4); af2[3] = a_frag(abase, 2, 3, lane); bf2[0] = b_frag_j<KIND, 2>(P.raw, P.S, 0); DQ_PIN();
-    DQ_MF(af1, bf1, 5); if constexpr (!LAST) b_scales_j<KIND>(rn, T1, sn, 0); DQ_PIN();
-    DQ_MF(af1, bf1, 6); bf2[1] = b_frag_j<KIND, 2>(P.raw, P.S, 1); DQ_PIN();
-    DQ_MF(af1, bf1, 7); if constexpr (!LAST) b_scales_j<KIND>(rn, T1, sn, 1); DQ_PIN();
-    // slice 2
-    DQ_MF(af2, bf2, 0); af3[0] = a_frag(abase, 3, 0, lane); DQ_PIN();
-    DQ_MF(af2, bf2, 1); af3[1] = a_frag(abase, 3, 1, lane); DQ_PIN();
-    DQ_MF(af2, bf2, 2); af3[2] = a_frag(abase, 3, 2, lane); DQ_PIN();
-    DQ_MF(af2, bf2, 3); af3[3] = a_frag(abase, 3, 3, lane); DQ_PIN();
-    DQ_MF(af2, bf2, 4); bf3[0] = b_frag_j<KIND, 3>(P.raw, P.S, 0); DQ_PIN();
-    DQ_MF(af2, bf2, 5); if constexpr (!LAST) bn[0] = b_frag_j<KIND, 0>(rn, sn, 0); DQ_PIN();
-    DQ_MF(af2, bf2, 6); bf3[1] = b_frag_j<KIND, 3>(P.raw, P.S, 1); DQ_PIN();
-    DQ_MF(af2, bf2, 7); if constexpr (!LAST) bn[1] = b_frag_j<KIND, 0>(rn, sn, 1); DQ_PIN();
-    // the next step's stage, the barrier, the DMAs into this step's stage
+    if constexpr (LAST) wait_vm<b_wait<NWN, KIND>()>();
+    DQ_SLOT(P.af, P.bf, 0, 0, );
+    DQ_SLOT(P.af, P.bf, 0, 1, (b_raw_j<NWN, KIND>(braw, T1, wn, lane, rn, 0)));
+    DQ_SLOT(P.af, P.bf, 0, 2, );
+    DQ_SLOT(P.af, P.bf, 0, 3, );
+    DQ_SLOT(P.af, P.bf, 0, 4, );
+    DQ_SLOT(P.af, P.bf, 0, 5, (b_raw_j<NWN, KIND>(braw, T1, wn, lane, rn, 1)));
+    DQ_SLOT(P.af, P.bf, 0, 6, );
+    DQ_SLOT(P.af, P.bf, 0, 7, );
+    DQ_TAKE();
+    DQ_SLOT(afc, bfc, 1, 0, );
+    DQ_SLOT(afc, bfc, 1, 1, if constexpr (MINB) P.bm[0] = q4k_neg_mins(P.raw.hd[0], lane < 32));
+    DQ_SLOT(afc, bfc, 1, 2, );
+    DQ_SLOT(afc, bfc, 1, 3, if constexpr (MINB) P.bm[1] = q4k_neg_mins(P.raw.hd[1], lane < 32));
+    DQ_SLOT(afc, bfc, 1, 4, );
+    DQ_SLOT(afc, bfc, 1, 5, (b_scales_j<KIND>(rn, T1, sn, 0)));
+    DQ_SLOT(afc, bfc, 1, 6, );
+    DQ_SLOT(afc, bfc, 1, 7, (b_scales_j<KIND>(rn, T1, sn, 1)));
+    DQ_TAKE();
+    DQ_SLOT(afc, bfc, 2, 0, );
+    DQ_SLOT(afc, bfc, 2, 1, );
+    DQ_SLOT(afc, bfc, 2, 2, );
+    DQ_SLOT(afc, bfc, 2, 3, );
+    DQ_SLOT(afc, bfc, 2, 4, );
+    DQ_SLOT(afc, bfc, 2, 5, );
+    DQ_SLOT(afc, bfc, 2, 6, );
+    DQ_SLOT(afc, bfc, 2, 7, );
+    DQ_TAKE();
+    // the next step's stage, the barrier, then slice 3 with the DMAs
     wait_vm<mid_wait<NWN, KIND, NS, T>()>();
     dq_lds_barrier();
-    issue_a<NWN, KIND>(g, aring + astage * R::A_STAGE, a_next, wn, lane);
-    if constexpr (T == 0) issue_b<NWN, KIND, TL>(g, bring + (b_next % NB) * R::B_STAGE, b_next, wn, lane);
-    DQ_PIN();
-    // slice 3
-    DQ_MF(af3, bf3, 0); P.af[0] = a_frag(anext, 0, 0, lane); DQ_PIN();
-    DQ_MF(af3, bf3, 1); P.af[1] = a_frag(anext, 0, 1, lane); DQ_PIN();
-    DQ_MF(af3, bf3, 2); P.af[2] = a_frag(anext, 0, 2, lane); DQ_PIN();
-    DQ_MF(af3, bf3, 3); P.af[3] = a_frag(anext, 0, 3, lane); DQ_PIN();
-    DQ_MF(af3, bf3, 4); if constexpr (LAST) b_raw_j<NWN, KIND>(bnext, 0, wn, lane, P.raw, 0); DQ_PIN();
-    DQ_MF(af3, bf3, 5); if constexpr (LAST) b_raw_j<NWN, KIND>(bnext, 0, wn, lane, P.raw, 1); DQ_PIN();
-    DQ_MF(af3, bf3, 6);
-    if constexpr (MINT) {
+    auto dma = [&](int q) {  // slot q's share of the PA + NBI instructions
+#pragma unroll
+        for (int i = q * PA / 8; i < (q + 1) * PA / 8; ++i)
+            dq_buf_lds<16>(src.a, aring + astage * R::A_STAGE + (i * NWN + wn) * 64 * 16, src.av[i],
+                           (uint32_t)(a_next * BK * 2));
+    };
+    auto dmb = [&](int q) {
+#pragma unroll
+        for (int i = q * NBI / 8; i < (q + 1) * NBI / 8; ++i)
+            issue_b1<NWN, KIND, TL>(g, src, bdst, b_next, wn, lane, b_first<KIND, T>() + i);
+    };
+#define DQ_SLOT3(Q, W)                                                                                \
+    DQ_MF(afc, bfc, Q);                                                                               \
+    if constexpr ((Q) % 2 == 0) P.af[(Q) / 2] = a_frag(anext, 0, (Q) / 2, lane);                      \
+    tw[(Q) / 4][(Q) % 4] = b_word<KIND, 0, (Q) % 4>(rn, sn, (Q) / 4, v);                              \
+    W;                                                                                                \
+    DQ_PIN()
+    // the A instructions first: a step's wait counts the B part after them
+    DQ_SLOT3(0, dma(0); dma(1));
+    DQ_SLOT3(1, dma(2); dma(3));
+    DQ_SLOT3(2, dma(4); dma(5));
+    DQ_SLOT3(3, dma(6); dma(7));
+    DQ_SLOT3(4, dmb(0); dmb(1));
+    DQ_SLOT3(5, dmb(2); dmb(3));
+    DQ_SLOT3(6, dmb(4); dmb(5); if constexpr (MINT) {
         am[0] = lds_h8(bbase + R::MIN + (0 * 32 + (lane & 31)) * 16);
         am[1] = lds_h8(bbase + R::MIN + (1 * 32 + (lane & 31)) * 16);
-    }
-    DQ_PIN();
-    DQ_MF(af3, bf3, 7);
-    if constexpr (MINT) {
+    });
+    DQ_SLOT3(7, dmb(6); dmb(7); if constexpr (MINT) {
         am[2] = lds_h8(bbase + R::MIN + (2 * 32 + (lane & 31)) * 16);
         am[3] = lds_h8(bbase + R::MIN + (3 * 32 + (lane & 31)) * 16);
-    }
-    DQ_PIN();
+    });
     if constexpr (MINT) {
         // the super-block's min term: the block sums (lanes 0-31: the 8 K
-        // values; lanes 32-63 zero) against -dmin*m; the next super-stage's
-        // B side is converted behind it
-        const h8 zero = {};
+        // values) against -dmin*m, which lanes 32-63 hold as zeros
 #pragma unroll
-        for (int i = 0; i < 4; ++i) am[i] = (lane >> 5) == 0 ? am[i] : zero;
-        DQ_MF(am, P.bm, 0); b_scales_j<KIND>(P.raw, 0, P.S, 0); DQ_PIN();
-        DQ_MF(am, P.bm, 1); DQ_PIN();
-        DQ_MF(am, P.bm, 2); b_scales_j<KIND>(P.raw, 0, P.S, 1); DQ_PIN();
-        DQ_MF(am, P.bm, 3); DQ_PIN();
-        DQ_MF(am, P.bm, 4); P.bf[0] = b_frag_j<KIND, 0>(P.raw, P.S, 0); DQ_PIN();
-        DQ_MF(am, P.bm, 5); DQ_PIN();
-        DQ_MF(am, P.bm, 6); P.bf[1] = b_frag_j<KIND, 0>(P.raw, P.S, 1); DQ_PIN();
-        DQ_MF(am, P.bm, 7); DQ_PIN();
-    } else if constexpr (LAST) {
-        b_scales<KIND>(P.raw, 0, P.S);
-        b_frag<KIND, 0>(P.raw, P.S, P.bf);
-    } else {
-        P.raw = rn;
-        P.S = sn;
-        P.bf[0] = bn[0];
-        P.bf[1] = bn[1];
+        for (int q = 0; q < 8; ++q) DQ_MF(am, P.bm, q);
     }
+    P.raw = rn;
+    P.S = sn;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) P.bf[j] = __builtin_bit_cast(h8, dq_u32x4{tw[j][0], tw[j][1], tw[j][2], tw[j][3]});
     astage = next_stage;
 }
+#undef DQ_SLOT3
+#undef DQ_TAKE
+#undef DQ_SLOT
 #undef DQ_MF
 #undef DQ_PIN
 
@@ -585,12 +631,24 @@ __device__ __forceinline__ void run_steps(const GemmArgs& g, uint8_t* aring, uin
     constexpr int SB = R::SB, NB = R::NB, PA = a_loads<NWN>(), PB = b_loads<KIND>();
     if (sb0 >= sb1) return;  // uniform over the workgroup (the planner gives every K group the same count)
     const int s0 = SB * sb0, s_last = SB * sb1 - 1, sb_last = sb1 - 1;
-    issue_b<NWN, KIND, TL>(g, bring + (sb0 % NB) * R::B_STAGE, sb0, wn, lane);
-    issue_a<NWN, KIND>(g, aring, s0, wn, lane);
-    issue_a<NWN, KIND>(g, aring + R::A_STAGE, min(s0 + 1, s_last), wn, lane);
-    if constexpr (NB == 3)
-        issue_b<NWN, KIND, TL>(g, bring + ((sb0 + 1) % NB) * R::B_STAGE, min(sb0 + 1, sb_last), wn, lane);
-    if constexpr (NS == 3) issue_a<NWN, KIND>(g, aring + 2 * R::A_STAGE, min(s0 + 2, s_last), wn, lane);
+    Src<NWN, KIND> src;
+    make_src<NWN, KIND, TL>(g, wn, lane, src);
+    issue_b<NWN, KIND, TL>(g, src, bring + (sb0 % NB) * R::B_STAGE, sb0, wn, lane);
+    // A(s0 + k) and, NB = 3, the halves of B(sb0 + 1) in the order the steps
+    // -NS .. -1 would have issued them (the waits count on it)
+    auto b_half = [&](int h) {
+        const int lo = h ? b_loads<KIND>() / 2 : 0, hi = h ? b_loads<KIND>() : b_loads<KIND>() / 2;
+#pragma unroll
+        for (int i = 0; i < b_loads<KIND>(); ++i)
+            if (i >= lo && i < hi)
+                issue_b1<NWN, KIND, TL>(g, src, bring + ((sb0 + 1) % NB) * R::B_STAGE, min(sb0 + 1, sb_last), wn, lane, i);
+    };
+    issue_a<NWN, KIND>(src, aring, s0, wn);
+    if constexpr (NB == 3 && NS == 2) b_half(0);
+    issue_a<NWN, KIND>(src, aring + R::A_STAGE, min(s0 + 1, s_last), wn);
+    if constexpr (NB == 3) b_half(NS == 2 ? 1 : 0);
+    if constexpr (NS == 3) issue_a<NWN, KIND>(src, aring + 2 * R::A_STAGE, min(s0 + 2, s_last), wn);
+    if constexpr (NB == 3 && NS == 3) b_half(1);
     // wait for B(sb0) and A(s0): the loads issued after A(s0) may stay in flight
     wait_vm<(NS - 1) * PA + (NB == 3 ? PB : 0)>();
     dq_lds_barrier();
@@ -604,11 +662,11 @@ __device__ __forceinline__ void run_steps(const GemmArgs& g, uint8_t* aring, uin
     for (int sb = sb0; sb < sb1; ++sb) {
         const int st = SB * sb;
         const int bn = min(sb + NB - 1, sb_last);
-        gemm_step<NWN, KIND, NS, 0, TL>(g, aring, bring, astage, sb, min(st + NS, s_last), bn, P, acc, wn, lane);
-        gemm_step<NWN, KIND, NS, 1, TL>(g, aring, bring, astage, sb, min(st + 1 + NS, s_last), bn, P, acc, wn, lane);
+        gemm_step<NWN, KIND, NS, 0, TL>(g, src, aring, bring, astage, sb, min(st + NS, s_last), bn, P, acc, wn, lane);
+        gemm_step<NWN, KIND, NS, 1, TL>(g, src, aring, bring, astage, sb, min(st + 1 + NS, s_last), bn, P, acc, wn, lane);
         if constexpr (SB == 4) {
-            gemm_step<NWN, KIND, NS, 2, TL>(g, aring, bring, astage, sb, min(st + 2 + NS, s_last), bn, P, acc, wn, lane);
-            gemm_step<NWN, KIND, NS, 3, TL>(g, aring, bring, astage, sb, min(st + 3 + NS, s_last), bn, P, acc, wn, lane);
+            gemm_step<NWN, KIND, NS, 2, TL>(g, src, aring, bring, astage, sb, min(st + 2 + NS, s_last), bn, P, acc, wn, lane);
+            gemm_step<NWN, KIND, NS, 3, TL>(g, src, aring, bring, astage, sb, min(st + 3 + NS, s_last), bn, P, acc, wn, lane);
         }
     }
     wait_vm<0>();  // drain the DMAs issued past the end
@@ -695,31 +753,33 @@ void gemm_kernel(GemmArgs g, float* __restrict__ y, int nsb, int sb_per_split, i
             }
             __syncthreads();
         }
-        if (kg != 0) return;
     }
 
     // D layout of 32x32x16: lane l, register r -> n = l%32, m = (r/4)*8 + (l/32)*4 + r%4.
-    // The row factors 1/s of a 32-token block are loaded together before its
-    // stores (unconditional loads of clamped rows; a load inside the store's
-    // branch would be waited for one at a time).
+    // The row factors 1/s go through the (drained) ring: 16 dependent loads
+    // per 32-token block from memory would be four more round trips. The
+    // outputs are written past the caches (they are read by another kernel,
+    // often from another XCD): the write-back of dirty lines at the kernel's
+    // end is 2 us at 29 MB of output.
+    float* sinv = reinterpret_cast<float*>(ring);
+    if (tid < BM) sinv[tid] = g.inv[min(g.m0 + tid, g.M - 1)];
+    __syncthreads();
+    if (kg != 0) return;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int mb0 = g.m0 + i * 32 + (lane >> 5) * 4;
-        float inv[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) inv[r] = g.inv[min(mb0 + (r >> 2) * 8 + (r & 3), g.M - 1)];
+        const int ml0 = i * 32 + (lane >> 5) * 4;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = g.n0 + wn * 64 + j * 32 + (lane & 31);
             if (n >= g.N) continue;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m = mb0 + (r >> 2) * 8 + (r & 3);
-                if (m < g.M) {
-                    float* dst = y + (size_t)m * g.N + n;
-                    const float v = acc[i][j][r] * inv[r];  // a power of two: exact
+                const int ml = ml0 + (r >> 2) * 8 + (r & 3);
+                if (g.m0 + ml < g.M) {
+                    float* dst = y + (size_t)(g.m0 + ml) * g.N + n;
+                    const float v = acc[i][j][r] * sinv[ml];  // a power of two: exact
                     if (atomic_out) atomicAdd(dst, v);
-                    else *dst = v;
+                    else __builtin_nontemporal_store(v, dst);
                 }
             }
         }
@@ -1152,10 +1212,15 @@ static int launch_gemm(const GemmArgs& g, size_t rows, size_t n_tok, int nsb, in
 // for Q8_0, whose B super-stages leave no room for a second ring), optionally
 // with a 2-way K split over workgroups (two partials added atomically into
 // zeroed y: a+b == b+a, so the result is deterministic). One workgroup per
-// CU; the plan with the fewest super-blocks on the busiest CU wins (rounds of
-// the grid times super-blocks per K group), ties going to no split and then
-// to 4x1. DQ_GEMM_SHAPE (41 or 22) and DQ_GEMM_SPLIT (1 or 2) override it for
-// tuning where the override is valid.
+// CU. The plan with the least estimated time wins (rounds of the grid times
+// super-blocks per K group, at what one super-block takes with every CU at
+// work, plus the second partial's additions), ties going to no split and then
+// to 4x1. Measured, us: a super-block 3.5 for 4x1 and 4.3 for 2x2 (half the
+// rows per activation fragment read), the additions 1.5 per MB of y. Q4_K
+// 14336 x 4096 at 2048 tokens takes 287 as 4x1 and 330 as 2x2 (an equal count
+// of super-blocks), Q6_K 4096 x 14336 at 512 tokens 102 as 2x2 split and 134
+// as 4x1 split. DQ_GEMM_SHAPE (41 or 22) and DQ_GEMM_SPLIT (1 or 2) override
+// it for tuning where the override is valid.
 struct GemmPlan {
     int nwn, split;
 };
@@ -1175,7 +1240,9 @@ static GemmPlan plan_gemm(int fmt, size_t rows, size_t n_tok, int nsb, int cu_bu
             const int ksw = 4 / nwn;
             const size_t wgs = mb * ((rows + 64 * nwn - 1) / (64 * nwn)) * split;
             const int per_split = (nsb + split - 1) / split;
-            const size_t cost = ((wgs + c - 1) / c) * (size_t)((per_split + ksw - 1) / ksw);
+            const size_t units = ((wgs + c - 1) / c) * (size_t)((per_split + ksw - 1) / ksw);
+            const size_t cost = units * (nwn == 4 ? 3500 : 4300) +
+                                (split == 2 ? (size_t)(rows * n_tok * 4 * 1.5e-3) : 0);  // ns
             if (cost < best_cost) {
                 best_cost = cost;
                 best = GemmPlan{nwn, split};
