@@ -41,6 +41,7 @@
 
 #include "dq_common.h"
 #include "dq_f16.h"
+#include "dq_moe_tiles.h"
 
 namespace {
 
@@ -562,9 +563,9 @@ __device__ __forceinline__ void issue_a(const ASrc& s, int n_pairs, int st, uint
 // HBM streams at full rate; one lane per row, 16 bytes each, streams at less
 // than half of it). Item t of row r sits in chunk slot t ^ ((r >> 2) & 3), so
 // the fragment reads of 32 rows spread over the banks.
-constexpr int WROWS = 32 * WAVES;                  // rows per workgroup
+static_assert(WROWS == 32 * WAVES, "rows per workgroup");
 constexpr int WT_PLANE = WROWS * 64;               // bytes of one sub-plane tile
-constexpr int WT_BYTES = 2 * WT_PLANE + WROWS * 16;
+static_assert(WT_BYTES == 2 * WT_PLANE + WROWS * 16, "tile bytes");
 __device__ __forceinline__ void issue_w(const uint8_t* base, const DqLayout& L, size_t row0, int nrows, int st,
                                         uint8_t* dst, int tid) {
     const int wbase = tid & ~63;
@@ -588,14 +589,11 @@ __device__ __forceinline__ void issue_w(const uint8_t* base, const DqLayout& L, 
 }
 static_assert(WROWS * 4 % (64 * WAVES) == 0 && 64 * WAVES == 2 * WROWS, "DMA slots per thread");
 
-// Expert-tile layout (DQ_FMT_Q4_K_TILES): the weight tile of one main step
-// stored as the LDS stage image, so the step's DMA reads one contiguous
-// run (64 lanes x 16 consecutive bytes per instruction) instead of 4 lanes
-// per 64-byte row piece. Chunk (e, x, sb) of expert e, row tile x (rows
-// 128x .. +127, the last row repeated past the expert's end) and super-block
-// sb sits at ((e * n_tiles + x) * nsb + sb) * WT_BYTES: the two sub-plane
-// tiles [128 rows][4 slots][16 B] (slot t ^ ((r >> 2) & 3) holding item t)
-// and the headers [128 rows][16 B].
+// Expert tiles (DQ_FMT_Q4_K_TILES, dq_moe_tiles.h): the step's DMA copies one
+// contiguous run into the LDS stage (64 lanes x 16 consecutive bytes per
+// instruction) instead of 4 lanes per 64-byte row piece. Chunk (e, x, sb) of
+// expert e, row tile x and super-block sb sits at ((e * n_tiles + x) * nsb +
+// sb) * WT_BYTES.
 constexpr int WT_SLOTS = WT_BYTES / 16;
 constexpr int WT_TILE_LOADS = (WT_SLOTS + 64 * WAVES - 1) / (64 * WAVES);  // DMAs per thread per step
 static_assert(WT_TILE_LOADS == 2 * WROWS * 4 / (64 * WAVES) + 1, "the same DMA count as the row layout");
@@ -615,25 +613,27 @@ __device__ __forceinline__ void issue_w_tiles(const uint8_t* chunk, uint8_t* dst
 __global__ __launch_bounds__(256) void moe_tiles_pack_kernel(const uint8_t* __restrict__ src, DqLayout L, int rows,
                                                              int n_tiles, int nsb, size_t n_slots,
                                                              uint8_t* __restrict__ dst) {
-    const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (g >= n_slots) return;
-    const size_t chunk = g / WT_SLOTS;
-    const int c = (int)(g % WT_SLOTS);
+    const size_t s = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (s >= n_slots) return;
+    const size_t chunk = s / (WT_BYTES / 16);
+    const int c = (int)(s % (WT_BYTES / 16)), grp = c / (WG_BYTES / 16), q = c % (WG_BYTES / 16);
     const int sb = (int)(chunk % nsb);
     const size_t et = chunk / nsb;
     const int x = (int)(et % n_tiles);
     const size_t e = et / n_tiles;
-    const uint8_t* p;
-    if (c < 2 * WROWS * 4) {
-        const int pl = c / (WROWS * 4), rs = c % (WROWS * 4), r = rs / 4, t = (rs % 4) ^ ((r >> 2) & 3);
-        const size_t row = e * rows + (size_t)min(WROWS * x + r, rows - 1);
-        p = src + L.q_off + (size_t)pl * L.p_stride + row * L.q_row + 16 * (size_t)(4 * sb + t);
+    const int n = q < 128 ? q & 15 : q - 128;
+    const size_t row = e * rows + (size_t)min(WROWS * x + 16 * grp + n, rows - 1);
+    dq_u32x4 v;
+    if (q < 128) {
+        const int i = q >> 6, g = (q >> 4) & 3;
+        const uint8_t* p = src + L.q_off + (size_t)(g >> 1) * L.p_stride + row * L.q_row + 64 * (size_t)sb + 32 * i +
+                           8 * (g & 1);
+        const dq_u32x2 a = *reinterpret_cast<const dq_u32x2*>(p), b = *reinterpret_cast<const dq_u32x2*>(p + 16);
+        v = dq_u32x4{a.x, a.y, b.x, b.y};
     } else {
-        const int r = c - 2 * WROWS * 4;
-        const size_t row = e * rows + (size_t)min(WROWS * x + r, rows - 1);
-        p = src + L.s_off + row * L.s_row + 16 * (size_t)sb;
+        v = *reinterpret_cast<const dq_u32x4*>(src + L.s_off + row * L.s_row + 16 * (size_t)sb);
     }
-    *reinterpret_cast<dq_u32x4*>(dst + 16 * g) = *reinterpret_cast<const dq_u32x4*>(p);
+    *reinterpret_cast<dq_u32x4*>(dst + 16 * s) = v;
 }
 
 size_t tiles_bytes(size_t n_exp, size_t rows, size_t cols) {
@@ -729,11 +729,25 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
                 // every LDS read of the step first (one wait for all of them),
                 // then the dequantization and the MFMAs
                 WRaw wr;
+                if constexpr (TILED) {
+                    // slots (n, 2h) and (n, 2h + 1) of run i: the two halves of
+                    // sub-plane h of items 2i (first 8 bytes) and 2i + 1
+                    const uint8_t* gb = wb + (rl >> 4) * WG_BYTES + (rl & 15) * 16;
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    wr.q[t] = *reinterpret_cast<const dq_u32x4*>(wb + h * WT_PLANE + rl * 64 +
-                                                                 16 * (t ^ ((rl >> 2) & 3)));
-                wr.hd = *reinterpret_cast<const dq_u32x4*>(wb + 2 * WT_PLANE + rl * 16);
+                    for (int i = 0; i < 2; ++i) {
+                        const dq_u32x4 a = *reinterpret_cast<const dq_u32x4*>(gb + 1024 * i + h * 512);
+                        const dq_u32x4 b = *reinterpret_cast<const dq_u32x4*>(gb + 1024 * i + h * 512 + 256);
+                        wr.q[2 * i] = dq_u32x4{a.x, a.y, b.x, b.y};
+                        wr.q[2 * i + 1] = dq_u32x4{a.z, a.w, b.z, b.w};
+                    }
+                    wr.hd = *reinterpret_cast<const dq_u32x4*>(gb + 2048);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        wr.q[t] = *reinterpret_cast<const dq_u32x4*>(wb + h * WT_PLANE + rl * 64 +
+                                                                     16 * (t ^ ((rl >> 2) & 3)));
+                    wr.hd = *reinterpret_cast<const dq_u32x4*>(wb + 2 * WT_PLANE + rl * 16);
+                }
                 const int m = lane & 31;
                 h8 af[4][4];
 #pragma unroll
@@ -805,6 +819,7 @@ struct MoeWs {
     float *wts, *inv_in, *inv_h;
     _Float16 *a_in, *a_h, *min_in, *min_h;
     float *gate, *up, *down;
+    uint8_t* few;
     size_t total;
 };
 
@@ -845,6 +860,8 @@ MoeWs carve(const dq_moe_t* m, uint32_t n_tok, int split_gu, int split_d, uint8_
     w.offsets = (int32_t*)take((m->n_expert + 1) * 4);
     w.pairs = (int32_t*)take(n_ent * 4);
     w.slot_pos = (int32_t*)take(n_ent * 4);
+    w.few = base ? base + off : nullptr;  // the few-token form's buffers, in place of the rest
+    const size_t few_end = dq_moe_few(m->n_expert, n_ent) ? off + dq_moe_few_bytes(m, n_ent) : 0;
     w.inv_in = (float*)take(n_ent * 4);
     w.inv_h = (float*)take((size_t)split_d * n_ent * 4);
     w.a_in = (_Float16*)take(n_ent * E * 2);
@@ -854,7 +871,7 @@ MoeWs carve(const dq_moe_t* m, uint32_t n_tok, int split_gu, int split_d, uint8_
     w.a_h = (_Float16*)take(n_ent * F * 2);
     w.min_h = (_Float16*)take(n_ent * (F / 32) * 2);
     w.down = (float*)take((size_t)split_d * n_ent * E * 4);
-    w.total = off;
+    w.total = off > few_end ? off : few_end;
     return w;
 }
 
@@ -986,6 +1003,14 @@ int dq_moe_ffn(const dq_moe_t* m, const float* d_x, const float* d_logits, uint3
         DQ_TRY(dq_launch_status());
         moe_lists_kernel<<<1, 256, 0, s>>>(w.ids, n_ent, n_exp, w.offsets, w.pairs, w.slot_pos);
         DQ_TRY(dq_launch_status());
+    }
+    if (dq_moe_few(m->n_expert, (size_t)n_ent)) {
+        float* down = nullptr;
+        DQ_TRY(dq_moe_few_ffn(m, d_x, w.pairs, w.offsets, (size_t)n_ent, &down, w.few, s));
+        const size_t n = (size_t)n_tok * E;
+        moe_scatter_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(down, 1, 0, w.slot_pos, w.wts, k, (int)n_tok, E,
+                                                                       d_out);
+        return dq_launch_status();
     }
     // activation rows of the pairs, each with its range scale
     if (E / 256 <= 4 * ACT_RB)
