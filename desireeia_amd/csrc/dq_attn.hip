@@ -7,9 +7,9 @@
 // position at 8 KV heads. Head dims 64, 128 and 256 are supported.
 //
 // Attention is split over positions (flash-decoding): a workgroup per (KV
-// head, tile of 64 positions) keeps the tile's max / sum / weighted V sum for
-// the query heads that share the KV head (GQA), and a merge kernel combines
-// the tiles and can quantize the output for the output projection (the kernel
+// head, run of positions) keeps the run's max / sum / weighted V sum for the
+// query heads that share the KV head (GQA), and a merge kernel combines the
+// runs and can quantize the output for the output projection (the kernel
 // boundary makes the records of every XCD visible without a device-wide cache
 // writeback per workgroup). The position may be read from device
 // memory at run time, so the same launch can be replayed in a graph for
@@ -23,6 +23,8 @@
 // bits; the int8 factors are exact) and fp32 sums in another order than the
 // reference's (which sums the softmax denominator in double); results agree
 // to ~1e-6 relative over any range of K / V scales.
+#include <algorithm>
+#include <climits>
 #include <cstdlib>
 #include <mutex>
 #include <type_traits>
@@ -32,8 +34,11 @@
 
 namespace {
 
-constexpr int TP = 64;         // positions per tile
+constexpr int TP = 64;         // positions per tile (and per record of the work area, at least)
 constexpr int NT = 256;        // threads per workgroup
+constexpr int PW = 32;         // positions of a wave's step
+constexpr int UP = PW * (NT / 64);  // positions of a workgroup's step
+static_assert(TP == 1 << 6 && UP == 1 << 7, "AttnArgs::unit_log2");
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 
@@ -85,36 +90,55 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const float* __restrict__
 }
 
 // ------------------------------------------------------------ attention --
-// One workgroup per (KV head, tile of TP positions): the tile's K and V rows
-// go straight into LDS (dword DMA), and the HPK query heads that share the KV
-// head (GQA: each KV byte is read once for all of them) are scored, the tile
-// softmax taken and the weighted V sum formed on the matrix cores; the
-// workgroup writes a partial record (acc[HD], tile max, tile sum) per head
-// for attn_merge_kernel.
+// One workgroup per (KV head, run of positions); its four waves take 32
+// positions a step each, in turn, and never wait for one another inside the
+// run: a wave moves its K and V rows into its own part of the LDS (16-byte
+// DMA), scores them for the HPK query heads that share the KV head (GQA: each
+// KV byte is read once for all of them), and adds the weighted V rows to its
+// own running maximum, sum and output; K of its next step is fetched as soon
+// as the scores are done, V after the V product. At the end the four states
+// are combined and the workgroup writes one record (acc[HD], max, sum) per
+// head for attn_merge_kernel.
 //
-// Both products run as v_mfma_f32_16x16x32_f16 with exact operands:
-//  * scores, per (16 positions, Q8_0 block b): A = the query's 32 values of
-//    block b (rows = heads), B = the 32 K bytes of each position (int8 values
-//    are exact in fp16); the fp32 result is scaled by the position's block
-//    scale dk and summed over the blocks, as the reference's
-//    sum_b dk * sum(q * k8);
-//  * weighted sum, per (32 positions, 16 dims of block b): A = the weight
-//    w[h][p] * dv[p][b] (rows = heads), B = the V bytes, read position-major.
-// The fp32 A operands are split into fp16 hi + lo parts (hi*B + lo*B: ~22
+// Both products run as v_mfma_f32_16x16x32_f16 with exact operands, positions
+// (then output dims) as rows and heads as columns:
+//  * scores, per (16 positions, Q8_0 block b): A = the 32 K bytes of each
+//    position (int8 values are exact in fp16), B = the query's 32 values of
+//    block b; the fp32 result is scaled by the position's block scale dk and
+//    summed over the blocks, as the reference's sum_b dk * sum(q * k8);
+//  * weighted sum, per (32 positions, 16 dims of block b): A = the V bytes
+//    (lane n16 takes dims 2 n16 and 2 n16 + 1 of the block, one halfword per
+//    position, for two products), B = the weight w[h][p] * dv[p][b]. The
+//    scores of two 16-position products are in exactly the lanes that the
+//    B operand wants them in, with operand slot 8 g4 + j as position
+//    16 (j / 4) + 4 g4 + j % 4, so the weights never leave their registers.
+// The fp32 B operands are split into fp16 hi + lo parts (A*hi + A*lo: ~22
 // significant bits), after scaling by a power of two that puts the largest
-// value of the head (query) or block (weights) in [2^13, 2^14): no fp16
+// value of the head (query) or block (V scales) in [2^13, 2^14): no fp16
 // overflow, full precision for the values that matter, and the scaling is
 // undone exactly afterwards.
 //
-// FUSE: q, k, v are the raw projections of the new token: every workgroup
-// applies the optional bias / QK-norm and RoPE to its query heads, and the
-// workgroup of the last tile (the one holding `pos`) also processes k and v,
+// What bounds it: instruction issue (about 600 a step of 32 positions) and,
+// at long contexts, the memory. A workgroup of four waves over one tile of 64
+// positions, with the softmax and its weights exchanged through LDS behind
+// barriers, took 25.1 us + 12.2 us in the merge of 512 records for 32768
+// positions, 32/8 heads of 128; this form takes 19.3 us + 4.0 us.
+//
+// Runs: once there are more steps than the workgroups that the GPU holds at a
+// time (AttnArgs::wg_limit), a workgroup takes several steps, which keeps its
+// query operands and leaves fewer records to merge. Two workgroups per CU:
+// with 1, 3 and 4 the same call takes 21.8 + 4.1, 20.2 + 4.3 and 19.8 + 5.5 us
+// (64-value heads 14.8 + 3.9, 13.1 + 3.9 and 12.6 + 5.2 us, 13.0 + 3.9 with 2).
+//
+// FUSE: q, k, v are the raw projections of the new token: every wave applies
+// the optional bias / QK-norm and RoPE to its query operands, and the
+// workgroup of the last run (the one holding `pos`) also processes k and v,
 // quantizes the new K and V rows of its KV head (kv_quantize_row), writes
 // them into the cache and uses them directly. This replaces the separate
 // RoPE + KV-write kernel of the decoder layer.
 //
 // XCD-aware placement: consecutive workgroups go to different XCDs; the KV
-// heads of one tile share an XCD, so the 1088-byte position rows they split
+// heads of one run share an XCD, so the 1088-byte position rows they split
 // between them are fetched into one L2.
 struct AttnArgs {
     const float* q;     // [n_head][HD]: rotated (plain) or raw (FUSE)
@@ -125,6 +149,8 @@ struct AttnArgs {
     uint8_t* vc;
     size_t pos_bytes;
     int n_kv, cc_start, pos_host, n_ctx, max_tiles;
+    int wg_limit;         // workgroups of all KV heads' runs wanted at most
+    int unit_log2;        // positions of a step of a run (UP), or of a tile (TP)
     const int* pos_dev;
     float scale;
     float* part;          // [n_kv][max_tiles][HPK][HD + 4]
@@ -163,6 +189,55 @@ __device__ __forceinline__ void split_hl(float x, _Float16& hi, _Float16& lo) {
     lo = (_Float16)(x - (float)hi);
 }
 
+// fp16 hi + lo parts of 8 floats.
+__device__ __forceinline__ void split_hl8(const float (&x)[8], h8& hi, h8& lo) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const f2v v = {x[2 * i], x[2 * i + 1]};
+        const h2 h = __builtin_convertvector(v, h2);
+        const f2v r = {v.x - (float)h.x, v.y - (float)h.y};
+        const h2 l = __builtin_convertvector(r, h2);
+        hi[2 * i] = h.x, hi[2 * i + 1] = h.y;
+        lo[2 * i] = l.x, lo[2 * i + 1] = l.y;
+    }
+}
+
+// 8 floats from a 4-byte aligned address.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
+    const f4u a = *reinterpret_cast<const f4u*>(p), b = *reinterpret_cast<const f4u*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = a[i], x[4 + i] = b[i];
+}
+
+// Exchange of 16-lane rows (1 of a with 0 of b, 3 with 2) and of 32-lane halves
+// (high of a with low of b): on two copies of a value each lane is left with
+// the value of its own row / half and of its neighbour's. The s_nop is the wait
+// that a VALU result read by these needs.
+__device__ __forceinline__ void swap16(float& a, float& b) {
+    asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+
+// Maximum / sum over the four 16-lane rows of a wave, column by column.
+__device__ __forceinline__ float rows_max(float a) {
+    float b = a;
+    swap16(a, b);
+    a = b = fmaxf(a, b);
+    swap32(a, b);
+    return fmaxf(a, b);
+}
+__device__ __forceinline__ float rows_sum(float a) {
+    float b = a;
+    swap16(a, b);
+    a = b = a + b;
+    swap32(a, b);
+    return a + b;
+}
+
 // Exponent shift that brings a largest magnitude m into [2^13, 2^14) (0 for
 // m == 0 or not finite).
 __device__ __forceinline__ int pow2_shift(float m, int cap) {
@@ -172,6 +247,419 @@ __device__ __forceinline__ int pow2_shift(float m, int cap) {
     return min(14 - e, cap);
 }
 
+// Steps of a workgroup's run over n positions.
+__device__ __forceinline__ int run_steps(const AttnArgs& A, int n) {
+    const int units = (n + (1 << A.unit_log2) - 1) >> A.unit_log2;
+    const int wgs = units * A.n_kv;
+    return wgs <= A.wg_limit ? 1 : (wgs + A.wg_limit - 1) / A.wg_limit;
+}
+
+// LDS row of a position: RB bytes in 16-byte pieces, the last of which holds
+// the row's last 16 bytes, so that no piece reaches past the row.
+template <int HD>
+struct AttnRow {
+    static constexpr int NB = HD / 32;            // Q8_0 blocks
+    static constexpr int RB = NB * DQ_SZ_Q8_0;    // bytes
+    static constexpr int RBW = RB / 4;            // dwords
+    static constexpr int PIECES = (RBW + 3) / 4;
+    static constexpr int RWP = 4 * PIECES;        // dwords in LDS
+    static constexpr int RP = HD == 64 ? 1 : HD / 128;    // RoPE pairs per lane of a row
+    static constexpr int SHIFT = RWP - RBW;       // dwords from 4 (PIECES - 1) on are this much later
+    static constexpr int NDMA = (PW * PIECES + 63) / 64;  // DMA instructions of a step's rows
+    static constexpr int BUF = NDMA * 256;        // dwords of a step's rows in LDS
+    // workgroups of a CU in a grid that fills the GPU once (82 KB of LDS each
+    // for 256-value heads)
+    static constexpr int PER_CU = HD == 256 ? 1 : 2;
+};
+
+template <int HD, int HPK, bool FUSE>
+__global__ __launch_bounds__(NT, AttnRow<HD>::PER_CU) void attn_run_kernel(AttnArgs A) {
+    using R = AttnRow<HD>;
+    constexpr int NB = R::NB, RB = R::RB, RBW = R::RBW, RWP = R::RWP, NDMA = R::NDMA, BUF = R::BUF;
+    constexpr int NW = NT / 64;
+    constexpr int REC = HD + 4;            // acc[HD], max, sum, 2 pad (16-byte records)
+    constexpr int QV = HD / 64;            // values of a new row per lane (value lane + 64 i)
+    static_assert(dq_head_dim_ok<HD>() && HPK <= 8 && RB % 4 == 0 && HPK * HD <= 2 * BUF, "shape");
+
+    __shared__ __align__(16) uint32_t rows[NW][2][BUF];   // per wave: K and V rows of a step
+    __shared__ __align__(16) float scl[NW][2][NB * PW];   // and their block scales (V: times a power of two)
+    __shared__ uint32_t nrow[2][RBW];                     // FUSE: the new K and V rows
+    __shared__ float wm[NW][HPK], wl[NW][HPK];            // per wave: maximum and sum at the end
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n16 = lane & 15, g4 = lane >> 4;
+    const int n_xcd = 8;
+    const int xcd = blockIdx.x % n_xcd, slot = blockIdx.x / n_xcd;
+    const int kvh = slot % A.n_kv;
+    const int chunk = xcd + n_xcd * (slot / A.n_kv);
+    const int pos = read_pos(A.pos_host, A.pos_dev, A.n_ctx);
+    const int c0 = A.cc_start < pos ? A.cc_start : pos;
+    const int n = pos + 1 - c0;                    // positions
+    const int n_grp = (n + PW - 1) / PW;           // steps of all waves
+    const int span = NW * run_steps(A, n);
+    if (chunk * span >= n_grp || chunk >= A.max_tiles) return;
+    const int g_end = min(chunk * span + span, n_grp);
+    // the new row (position pos, the last row of the last run) is made here
+    const bool new_row = FUSE && g_end == n_grp;
+
+    // ---- the new K row (wave NW - 2) or V row (wave NW - 1), its bias, norm
+    // and RoPE table: value lane + 64 i. The last waves make them: they are the
+    // ones that have no step of their own when the run is short.
+    const int rw = wave - (NW - 2);
+    float xr[QV], br[QV], nr[QV], rc[R::RP], rs[R::RP];
+    if constexpr (FUSE) {
+        if (new_row && rw >= 0) {
+            const float* src = (rw == 0 ? A.k : A.v) + (size_t)kvh * HD + lane;
+            const float* bias = rw == 0 ? A.post.bk : A.post.bv;
+#pragma unroll
+            for (int i = 0; i < QV; ++i) {
+                xr[i] = src[64 * i];
+                br[i] = bias ? bias[(size_t)kvh * HD + lane + 64 * i] : 0.0f;
+                nr[i] = A.post.k_norm ? A.post.k_norm[lane + 64 * i] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < R::RP; ++i) {
+                const int j = HD == 64 ? (lane & 31) : lane + 64 * i;
+                rc[i] = A.rope ? A.rope[2 * j] : 1.0f;
+                rs[i] = A.rope ? A.rope[2 * j + 1] : 0.0f;
+            }
+        }
+    }
+    // ---- the query of head n16 (columns >= HPK repeat the last head and are
+    // never stored): values 32 b + 8 g4 + i, loaded ahead of the rows
+    const size_t hq = (size_t)kvh * HPK + min(n16, HPK - 1);
+    float x[NB][8], bq[NB][8], nq[NB][8], cs[NB / 2][2][8];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) load8(A.q + hq * HD + 32 * b + 8 * g4, x[b]);
+    if constexpr (FUSE) {
+        if (A.post.bq) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) load8(A.post.bq + hq * HD + 32 * b + 8 * g4, bq[b]);
+        }
+        if (A.post.q_norm) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) load8(A.post.q_norm + 32 * b + 8 * g4, nq[b]);
+        }
+        if (A.rope) {
+#pragma unroll
+            for (int b = 0; b < NB / 2; ++b) {
+                load8(A.rope + 2 * (32 * b + 8 * g4), cs[b][0]);
+                load8(A.rope + 2 * (32 * b + 8 * g4) + 8, cs[b][1]);
+            }
+        }
+    }
+    // ---- a step's K or V rows, straight into LDS: piece t of the buffer is
+    // piece t % PIECES of row t / PIECES. Rows past the last (under FUSE the
+    // new row too) are beyond the buffer's size and read as zeros: rows >= nv
+    // are never used, and the new row is written over afterwards.
+    uint32_t voff[NDMA];
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+        const int t = 64 * i + lane;
+        voff[i] = (uint32_t)(t / R::PIECES) * (uint32_t)A.pos_bytes + 4 * min(4 * (t % R::PIECES), RBW - 4);
+    }
+    auto fetch = [&](const uint8_t* cache, int which, int g) {
+        const int p0 = c0 + g * PW;
+        const int n_load = min(PW, pos + 1 - p0) - (FUSE && g == n_grp - 1 ? 1 : 0);
+        const __amdgpu_buffer_rsrc_t r = dq_buf(cache + (size_t)p0 * A.pos_bytes + (size_t)kvh * RB,
+                                                n_load > 0 ? (n_load - 1) * (uint32_t)A.pos_bytes + RB : 0);
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) dq_buf_lds<16>(r, &rows[wave][which][256 * i], voff[i], 0);
+    };
+    const int g0 = __builtin_amdgcn_readfirstlane(chunk * span + wave);
+    if (g0 < g_end) {
+        fetch(A.kc, 0, g0);
+        fetch(A.vc, 1, g0);
+    }
+    // ---- new K / V row (FUSE, last run): bias, K-norm and RoPE of k, then
+    // kv_quantize_row into nrow
+    if constexpr (FUSE) {
+        if (new_row && rw >= 0) {
+            if (rw == 0 ? A.post.bk : A.post.bv) {
+#pragma unroll
+                for (int i = 0; i < QV; ++i) xr[i] += br[i];
+            }
+            if (rw == 0 && A.post.k_norm) dq_head_rms_norm_w<HD>(xr, nr, A.post.eps);
+            if (rw == 0 && A.rope) {
+                if constexpr (HD == 64) {
+                    const float y = __shfl_xor(xr[0], 32, DQ_WAVE);
+                    xr[0] = lane < 32 ? xr[0] * rc[0] - y * rs[0] : y * rs[0] + xr[0] * rc[0];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < R::RP; ++i) {
+                        const float u = xr[i], w = xr[i + R::RP];
+                        xr[i] = u * rc[i] - w * rs[i];
+                        xr[i + R::RP] = u * rs[i] + w * rc[i];
+                    }
+                }
+            }
+            dq_q8_0_row<HD>(xr, lane, reinterpret_cast<uint8_t*>(nrow[rw]));
+        }
+    }
+    // ---- query operands: bias, QK-norm, RoPE (FUSE; NeoX pairs are HD / 2
+    // apart: block b and b + NB / 2 of one lane), then the head's power-of-two
+    // scale and the fp16 hi / lo split
+    h8 qh[NB], ql[NB];
+    float hs = 0.0f;
+    if (g0 < g_end) {
+        if constexpr (FUSE) {
+            if (A.post.bq) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[b][i] += bq[b][i];
+            }
+            if (A.post.q_norm) {
+                double s = 0.0;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) s += (double)(x[b][i] * x[b][i]);
+                s += __shfl_xor(s, 16, DQ_WAVE);
+                s += __shfl_xor(s, 32, DQ_WAVE);
+                const float sc = 1.0f / sqrtf((float)(s / (double)HD) + A.post.eps);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[b][i] = x[b][i] * sc * nq[b][i];
+            }
+            if (A.rope) {
+#pragma unroll
+                for (int b = 0; b < NB / 2; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float c = cs[b][i >> 2][2 * (i & 3)], s = cs[b][i >> 2][2 * (i & 3) + 1];
+                        const float u = x[b][i], w = x[b + NB / 2][i];
+                        x[b][i] = u * c - w * s;
+                        x[b + NB / 2][i] = u * s + w * c;
+                    }
+            }
+        }
+        float m = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(x[b][i]));
+        const int sh = pow2_shift(rows_max(m), 100);
+        const float sc = ldexpf(1.0f, sh);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = x[b][i] * sc;
+            split_hl8(y, qh[b], ql[b]);
+        }
+        hs = A.scale * ldexpf(1.0f, -sh);
+    }
+    if constexpr (FUSE) {
+        if (new_row) {  // workgroup-uniform
+            dq_lds_barrier();  // nrow
+            if (rw >= 0) {
+                const uint16_t* src = reinterpret_cast<const uint16_t*>(nrow[rw]);
+                uint16_t* grow = reinterpret_cast<uint16_t*>((rw == 0 ? A.kc : A.vc) + (size_t)pos * A.pos_bytes +
+                                                             (size_t)kvh * RB);
+                for (int l = lane; l < RB / 2; l += 64) grow[l] = src[l];
+            }
+        }
+    }
+    // ---- the run: this wave's steps
+    const uint32_t* const kt = rows[wave][0];
+    const uint8_t* const vb8 = reinterpret_cast<const uint8_t*>(rows[wave][1]);
+    float* const dks = scl[wave][0];
+    float* const dvs = scl[wave][1];
+    // dwords / bytes by which the lane's part of a row's last block is later
+    const int ksh = R::SHIFT && g4 == 3 ? R::SHIFT : 0;
+    constexpr int VS = (16 * (R::PIECES - 1) - (DQ_SZ_Q8_0 * (NB - 1) + 2)) / 2;
+    const int vsh = R::SHIFT && n16 >= VS ? 4 * R::SHIFT : 0;
+    float mr = -INFINITY, lr = 0.0f;   // running maximum of head n16, this lane's share of its sum
+    f4v oa[NB][2];                     // dims 32 b + 2 (4 g4 + r) + t of head n16
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) oa[b][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g = g0; g < g_end; g += NW) {  // wave-uniform
+        const int nv = min(PW, n - g * PW);
+        const bool more = g + NW < g_end;
+        // K has landed (the NDMA loads of V were issued after it)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+        if (FUSE && g == n_grp - 1) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            for (int l = lane; l < 2 * RWP; l += 64) {
+                const int w = l >= RWP, c = l - w * RWP;
+                rows[wave][w][(nv - 1) * RWP + c] = nrow[w][c < RWP - 4 ? c : c - R::SHIFT];
+            }
+        }
+        // block scales of K: [block][position]
+#pragma unroll
+        for (int i = 0; i < NB * PW / 64; ++i) {
+            const int p = (lane + 64 * i) / NB, b = lane % NB;
+            dks[b * PW + p] = dq_h2f(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(kt + p * RWP) +
+                                                                       DQ_SZ_Q8_0 * b));
+        }
+        // scores: rows 4 g4 + r of product gi are positions 16 gi + 4 g4 + r
+        f4v s[2] = {f4v{0.0f, 0.0f, 0.0f, 0.0f}, f4v{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+#pragma unroll
+            for (int gi = 0; gi < 2; ++gi) {
+                // quants of block b at row bytes 34 b + 2 + 8 g4 ...: dword
+                // aligned for odd b, two bytes in for even b (the last b is odd)
+                const uint32_t* kl = kt + (16 * gi + n16) * RWP + 2 * g4 + (b == NB - 1 ? ksh : 0);
+                constexpr int Z = DQ_SZ_Q8_0;
+                const int cb = (Z * b + 2) >> 2;
+                uint32_t w0, w1;
+                if (b & 1) {
+                    w0 = kl[cb];
+                    w1 = kl[cb + 1];
+                } else {
+                    const uint32_t d0 = kl[cb], d1 = kl[cb + 1], d2 = kl[cb + 2];
+                    w0 = __builtin_amdgcn_alignbyte(d1, d0, 2);
+                    w1 = __builtin_amdgcn_alignbyte(d2, d1, 2);
+                }
+                const h8 kv = i8x8_to_h8(w0, w1);
+                f4v c = {0.0f, 0.0f, 0.0f, 0.0f};
+                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, qh[b], c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, ql[b], c, 0, 0, 0);
+                const f4v dk = *reinterpret_cast<const f4v*>(dks + b * PW + 16 * gi + 4 * g4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[gi][r] = fmaf(dk[r], c[r], s[gi][r]);
+            }
+        }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the K rows are read
+            fetch(A.kc, 0, g + NW);
+        }
+        // softmax weights against the running maximum
+        float m = mr;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int p = 16 * (j >> 2) + 4 * g4 + (j & 3);
+            s[j >> 2][j & 3] = p < nv ? s[j >> 2][j & 3] * hs : -INFINITY;
+            m = fmaxf(m, s[j >> 2][j & 3]);
+        }
+        m = rows_max(m);
+        const float fr = __expf(mr - m);  // the first step: 0
+        mr = m;
+        float e[8];
+        float ls = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int p = 16 * (j >> 2) + 4 * g4 + (j & 3);
+            e[j] = p < nv ? __expf(s[j >> 2][j & 3] - m) : 0.0f;
+            ls += e[j];
+        }
+        lr = lr * fr + ls;
+        // V has landed (only K of the next step was issued after it)
+        if (more)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // block scales of V (0 past the positions) and their power of two:
+        // lanes of one block are NB apart
+        float inv;
+        {
+            float dv[NB * PW / 64];
+            float vm = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NB * PW / 64; ++i) {
+                const int p = (lane + 64 * i) / NB, b = lane % NB;
+                const float d = dq_h2f(*reinterpret_cast<const uint16_t*>(vb8 + p * RWP * 4 + DQ_SZ_Q8_0 * b));
+                dv[i] = p < nv ? d : 0.0f;
+                vm = fmaxf(vm, fabsf(dv[i]));
+            }
+            vm = fmaxf(vm, dq_dpp<0x128>(vm));                         // row_ror:8
+            if constexpr (NB <= 4) vm = fmaxf(vm, dq_dpp<0x124>(vm));  // row_ror:4
+            if constexpr (NB <= 2) vm = fmaxf(vm, dq_dpp<0x122>(vm));  // row_ror:2
+            const int sh = pow2_shift(rows_max(vm), 100);
+            const float sc = ldexpf(1.0f, sh);
+            inv = ldexpf(1.0f, -sh);
+#pragma unroll
+            for (int i = 0; i < NB * PW / 64; ++i) dvs[(lane % NB) * PW + (lane + 64 * i) / NB] = dv[i] * sc;
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            h8 ph, pl;
+            {
+                const f4v d0 = *reinterpret_cast<const f4v*>(dvs + b * PW + 4 * g4);
+                const f4v d1 = *reinterpret_cast<const f4v*>(dvs + b * PW + 16 + 4 * g4);
+                float y[8];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) y[j] = e[j] * d0[j], y[4 + j] = e[4 + j] * d1[j];
+                split_hl8(y, ph, pl);
+            }
+            const uint8_t* col = vb8 + 4 * g4 * RWP * 4 + DQ_SZ_Q8_0 * b + 2 + 2 * n16 + (b == NB - 1 ? vsh : 0);
+            const h2 k = {(_Float16)1152.0f, (_Float16)1152.0f};
+            dq_u32x4 v0, v1;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint8_t* c = col + (16 * (i >> 1) + 2 * (i & 1)) * RWP * 4;
+                const uint32_t w = (*reinterpret_cast<const uint16_t*>(c) |
+                                    (uint32_t)*reinterpret_cast<const uint16_t*>(c + RWP * 4) << 16) ^ 0x80808080u;
+                v0[i] = __builtin_bit_cast(uint32_t, magic_pair(w, 0x04020400u) - k);
+                v1[i] = __builtin_bit_cast(uint32_t, magic_pair(w, 0x04030401u) - k);
+            }
+            const float ib = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv), b));
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const h8 a = __builtin_bit_cast(h8, t ? v1 : v0);
+                f4v o = {0.0f, 0.0f, 0.0f, 0.0f};
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, o, 0, 0, 0);
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, o, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) oa[b][t][r] = fmaf(oa[b][t][r], fr, o[r] * ib);
+            }
+        }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the V rows are read
+            fetch(A.vc, 1, g + NW);
+        }
+    }
+    // ---- the four waves' states (a wave without positions: maximum -inf,
+    // the rest 0), through each wave's own rows, which it has read
+    {
+        float* st = reinterpret_cast<float*>(rows[wave][0]);
+        const float l = rows_sum(lr);
+        if (n16 < HPK) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    *reinterpret_cast<f4v*>(st + n16 * HD + 32 * b + 8 * g4 + 4 * q) =
+                        f4v{oa[b][0][2 * q], oa[b][1][2 * q], oa[b][0][2 * q + 1], oa[b][1][2 * q + 1]};
+            if (g4 == 0) {
+                wm[wave][n16] = mr;
+                wl[wave][n16] = l;
+            }
+        }
+    }
+    dq_lds_barrier();
+    float* rec = A.part + ((size_t)kvh * A.max_tiles + chunk) * HPK * REC;
+    for (int i = tid; i < HPK * HD / 4; i += NT) {
+        const int h = 4 * i / HD;
+        float M = wm[0][h];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) M = fmaxf(M, wm[w][h]);
+        f4v o = {0.0f, 0.0f, 0.0f, 0.0f};
+        float L = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float f = __expf(wm[w][h] - M);
+            const f4v v = reinterpret_cast<const f4v*>(rows[w][0])[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = fmaf(f, v[r], o[r]);
+            L = fmaf(f, wl[w][h], L);
+        }
+        float* d = rec + h * REC + 4 * i % HD;
+        *reinterpret_cast<f4v*>(d) = o;
+        if (4 * i % HD == 0) *reinterpret_cast<float2*>(rec + h * REC + HD) = make_float2(M, L);
+    }
+}
+
+// Short caches: one workgroup per (KV head, tile of 64 positions), each of the
+// four waves scoring 16 of the positions for all heads, the softmax weights of
+// the tile exchanged through LDS and the waves dividing the output dims; heads
+// as rows of both products. Query heads are prepared one per wave rather than
+// all by every wave, and there are twice as many, shorter workgroups.
 template <int HD, int HPK, bool FUSE>
 __global__ __launch_bounds__(NT) void attn_tile_kernel(AttnArgs A) {
     constexpr int NB = HD / 32;            // Q8_0 blocks per row
@@ -554,7 +1042,7 @@ __global__ __launch_bounds__(NT) void attn_tile_kernel(AttnArgs A) {
     }
 }
 
-// Merge of the tile records: workgroup b owns outputs [256b, 256b + 256) of
+// Merge of the records (here called tiles): workgroup b owns outputs [256b, 256b + 256) of
 // the flattened [n_head][HD] output (HD = 128: two heads). Thread (g, q)
 // takes output quad q (4 consecutive outputs, one 16-byte record load per
 // tile) and tiles g, g+MG, ... in batches of MB (all of a batch's record
@@ -581,7 +1069,9 @@ __global__ __launch_bounds__(MNT) void attn_merge_kernel(AttnArgs A) {
     const int g = tid / MQ, qd = tid % MQ;        // tile group, output quad
     const int pos = read_pos(A.pos_host, A.pos_dev, A.n_ctx);
     const int c0 = A.cc_start < pos ? A.cc_start : pos;
-    const int n_tiles = min((pos + 1 - c0 + TP - 1) / TP, A.max_tiles);
+    const int n_units = (pos + 1 - c0 + (1 << A.unit_log2) - 1) >> A.unit_log2;
+    const int run = run_steps(A, pos + 1 - c0);
+    const int n_tiles = min(run == 1 ? n_units : (n_units + run - 1) / run, A.max_tiles);  // records
     {
         const int ol = 4 * qd;                    // first output of the quad in the block
         const int hb = ol / HD;                   // head within the block
@@ -676,10 +1166,29 @@ size_t work_bytes_for(int n_head, int hd, int max_tiles) {
     return dq_align256((size_t)n_head * max_tiles * (hd + 4) * sizeof(float));
 }
 
+// Runs at most (attn_run_kernel): one per step of the cache, and beyond wg_limit
+// longer ones (run_steps keeps their number at ceil(wg_limit / n_kv)).
 template <int HD, int HPK, bool FUSE>
-int launch_attn(const AttnArgs& a, int n_head, hipStream_t st) {
-    const int slots = a.n_kv * ((a.max_tiles + 7) / 8);  // per XCD
-    attn_tile_kernel<HD, HPK, FUSE><<<8 * slots, NT, 0, st>>>(a);
+int launch_attn(AttnArgs a, int n_head, hipStream_t st) {
+    const int n_units = (a.n_ctx + UP - 1) / UP;
+    a.wg_limit = AttnRow<HD>::PER_CU * dq_gemm_cus();
+    // A cache that makes runs of one step only keeps to the tile kernel, which
+    // gives each wave half the positions and a quarter of the query work: 4097
+    // positions, 32/8 heads of 128, fused, 8.5 us and 8.6 by runs; 3134, 8/2
+    // heads of 256, the call 12.0 us and 12.5. Beyond it a run saves repeated
+    // query work, barriers and the merge's reads: 12104, 16/8 heads of 128, the
+    // call 15.3 us by tiles and 14.4 by runs; 32768, 32/8 heads, 25.1 + 12.2 and
+    // 19.3 + 4.0 us. The cache's size decides, not the position: that is on the
+    // device when a step is replayed.
+    if ((long)n_units * a.n_kv <= a.wg_limit) {
+        a.wg_limit = INT_MAX;
+        a.unit_log2 = 6;
+        attn_tile_kernel<HD, HPK, FUSE><<<8 * a.n_kv * ((a.max_tiles + 7) / 8), NT, 0, st>>>(a);
+    } else {
+        const int chunks = std::min(n_units, (a.wg_limit + a.n_kv - 1) / a.n_kv);
+        a.unit_log2 = 7;
+        attn_run_kernel<HD, HPK, FUSE><<<8 * a.n_kv * ((chunks + 7) / 8), NT, 0, st>>>(a);
+    }
     attn_merge_kernel<HD, HPK><<<n_head * HD / MNO, MNT, 0, st>>>(a);
     return dq_launch_status();
 }
