@@ -471,7 +471,9 @@ __global__ __launch_bounds__(NT, AttnRow<HD>::PER_CU) void attn_run_kernel(AttnA
     const int ksh = R::SHIFT && g4 == 3 ? R::SHIFT : 0;
     constexpr int VS = (16 * (R::PIECES - 1) - (DQ_SZ_Q8_0 * (NB - 1) + 2)) / 2;
     const int vsh = R::SHIFT && n16 >= VS ? 4 * R::SHIFT : 0;
-    float mr = -INFINITY, lr = 0.0f;   // running maximum of head n16, this lane's share of its sum
+    // running maximum of head n16 (finite from the start, so that positions that
+    // all score -inf weigh 0), this lane's share of its sum
+    float mr = -__FLT_MAX__, lr = 0.0f;
     f4v oa[NB][2];                     // dims 32 b + 2 (4 g4 + r) + t of head n16
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(NT, AttnRow<HD>::PER_CU) void attn_run_kernel(AttnA
             m = fmaxf(m, s[j >> 2][j & 3]);
         }
         m = rows_max(m);
-        const float fr = __expf(mr - m);  // the first step: 0
+        const float fr = __expf(mr - m);  // the first step: 0, or nothing to scale
         mr = m;
         float e[8];
         float ls = 0.0f;
@@ -614,7 +616,7 @@ __global__ __launch_bounds__(NT, AttnRow<HD>::PER_CU) void attn_run_kernel(AttnA
             fetch(A.vc, 1, g + NW);
         }
     }
-    // ---- the four waves' states (a wave without positions: maximum -inf,
+    // ---- the four waves' states (a wave without positions: the lowest maximum,
     // the rest 0), through each wave's own rows, which it has read
     {
         float* st = reinterpret_cast<float*>(rows[wave][0]);

@@ -66,3 +66,29 @@ def test_attention_runs(gpu, orc, hd, n_head, n_kv, pos, cc_start, fused):
     worst = max(rel(g, w) for g, w in zip(got, want))
     print(f"  worst head {worst:.2e}", flush=True)
     assert worst <= 1e-5
+
+
+@pytest.mark.parametrize("spans", [
+    [(0, 128)],                           # the first step of a run's four waves
+    [(800, 832), (1920, 2560)],           # a later step of one wave, a whole run
+])
+def test_attention_runs_minus_infinity(gpu, orc, spans):
+    """Positions whose scores are all -inf weigh 0, wherever the steps put them."""
+    hd, n_head, n_kv, pos = 128, 64, 32, 9000   # runs of 5 steps
+    print(f"attn runs -inf {spans}", flush=True)
+    kc, vc = host_cache(orc, pos + 1, n_kv, seed=7, hd=hd)
+    rng = np.random.default_rng(7)
+    q = rng.standard_normal(n_head * hd).astype(np.float32)
+    q.reshape(n_head, hd)[:, :32] = 1.0
+    blocks = kc.reshape(pos + 1, n_kv, hd // 32, 34)
+    keep = np.ones(pos + 1, bool)
+    for a, b in spans:
+        blocks[a:b, :, 0, :2] = np.array([np.inf], np.float16).view(np.uint8)
+        blocks[a:b, :, 0, 2:] = 255         # quants of -1
+        keep[a:b] = False
+    n_ctx = max(pos + 5, 128 * (2 * torch.cuda.get_device_properties(gpu).multi_processor_count // n_kv + 1))
+    got = ops.attention_decode(torch.from_numpy(q).to(gpu), device_cache(gpu, kc, vc, n_ctx, n_kv, hd=hd), n_head, pos, 0)
+    kept = [np.ascontiguousarray(c.reshape(pos + 1, -1)[keep]).reshape(-1) for c in (kc, vc)]
+    want = orc.attn_decode(q, *kept, n_head, n_kv, hd, 0, int(keep.sum()) - 1, f64=True)
+    got, want = got.cpu().numpy().reshape(n_head, hd), np.asarray(want).reshape(n_head, hd)
+    assert max(rel(g, w) for g, w in zip(got, want)) <= 1e-5
