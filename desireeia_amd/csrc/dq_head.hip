@@ -31,7 +31,7 @@
 namespace {
 
 constexpr int TK_CHUNK = 4096;  // keys per workgroup and pass
-constexpr int TK_T = 256;       // threads per workgroup
+constexpr int TK_T = 256;       // threads per workgroup of the kk = 1 pass
 
 __device__ __forceinline__ uint64_t order_key(float v, uint32_t id) {
     uint32_t u = __builtin_bit_cast(uint32_t, v == 0.0f ? 0.0f : v);
@@ -45,131 +45,141 @@ __device__ __forceinline__ float key_value(uint64_t k) {
     return __builtin_bit_cast(float, u);
 }
 
-constexpr int TK_PER = TK_CHUNK / TK_T;  // keys per thread
+constexpr int TK_S = 1024;               // threads per workgroup of the selection
+constexpr int TK_PER = TK_CHUNK / TK_S;  // its keys per thread
 
-// Sorts the first P (a power of two <= TK_CHUNK) keys of LDS ascending.
-__device__ void bitonic_sort(uint64_t* s, int P) {
-    for (int size = 2; size <= P; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int t = threadIdx.x; t < P / 2; t += TK_T) {
-                const int i = 2 * t - (t & (stride - 1)), j = i + stride;
-                const bool asc = (i & size) == 0;
-                const uint64_t a = s[i], b = s[j];
-                if ((a > b) == asc) {
-                    s[i] = b;
-                    s[j] = a;
-                }
-            }
-            __syncthreads();
-        }
-    }
+// Inclusive prefix sum over the wave.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
 }
 
 // One selection pass over chunk blockIdx.x (float logits with their index as
 // id on the first pass, keys afterwards): the kk smallest keys of the chunk.
-// Radix select: eight rounds of an 8-bit LDS histogram over the keys that
-// share the prefix fixed so far find the kk-th smallest key K exactly (keys
-// are distinct: the id is in them); the keys <= K are then gathered, and on
-// the final pass (one chunk) sorted.
-__global__ __launch_bounds__(TK_T) void topk_pass_kernel(const float* __restrict__ v, const uint64_t* __restrict__ kin,
+// Radix select: rounds of an 8-bit LDS histogram over the keys that share the
+// prefix fixed so far narrow down the kk-th smallest key, until all keys of
+// its bin are wanted (keys are distinct: the id is in them). The keys up to
+// the bin are then gathered, and on the final pass (one chunk) ordered.
+//
+// What bounds it: a chain of LDS round trips and barriers in few workgroups
+// (32 for 128256 logits, then one). So four keys a thread, a barrier per
+// round (a histogram per round, scanned by every wave for itself), one LDS
+// add per wave for its leading digit (the survivors of a first pass share
+// the top digits: one address for all adds), one position counter add per
+// wave, and the final order by counting smaller keys instead of sorting.
+// Norm, head product and 104 of 128256 logits: 101.9 -> 88.6 us against 256
+// threads of 16 keys, three barriers a round and a bitonic final sort.
+__global__ __launch_bounds__(TK_S) void topk_pass_kernel(const float* __restrict__ v, const uint64_t* __restrict__ kin,
                                                          uint32_t n, uint32_t kk, int sorted,
                                                          uint64_t* __restrict__ kout, int32_t* __restrict__ ids,
                                                          float* __restrict__ vals) {
-    __shared__ uint32_t hist[256];
+    __shared__ __align__(16) uint32_t hist[8][256];
     __shared__ uint64_t list[256];
-    __shared__ uint64_t s_prefix, s_key;
-    __shared__ uint32_t s_rank, s_cnt, s_bin;
-    const int t = threadIdx.x;
+    __shared__ uint32_t order[256];
+    __shared__ uint32_t s_cnt;
+    const int t = threadIdx.x, lane = t & 63;
     const size_t base = (size_t)blockIdx.x * TK_CHUNK;
     uint64_t key[TK_PER];
 #pragma unroll
     for (int j = 0; j < TK_PER; ++j) {
-        const size_t g = base + (size_t)j * TK_T + t;  // coalesced
+        const size_t g = base + (size_t)j * TK_S + t;  // coalesced
         uint64_t k = ~0ull;
         if (g < n) k = kin ? kin[g] : order_key(v[g], (uint32_t)g);
         key[j] = k;
     }
+    for (int i = t; i < 8 * 256; i += TK_S) hist[i / 256][i % 256] = 0;
+    if (t < 256) order[t] = 0, list[t] = ~0ull;
+    if (t == 0) s_cnt = 0;
+    __syncthreads();
     const size_t m = n - base < (size_t)TK_CHUNK ? n - base : (size_t)TK_CHUNK;  // keys in this chunk
     const uint32_t want = (uint32_t)(kk < m ? kk : m);
     uint64_t prefix = 0;
-    uint32_t rank = want;  // 1-based rank of K among the keys with this prefix
-    for (int r = 0; r < 8; ++r) {
-        const int shift = 56 - 8 * r;
-        hist[t] = 0;
-        __syncthreads();
+    uint32_t rank = want;  // 1-based rank of the want-th key among the keys with this prefix
+    int shift = 56;
+    bool whole = false;    // all keys with the prefix are wanted
+    for (int r = 0;; ++r, shift -= 8) {
 #pragma unroll
         for (int j = 0; j < TK_PER; ++j) {
             const bool match = r == 0 || (key[j] >> (shift + 8)) == prefix;
-            if (match) atomicAdd(&hist[(key[j] >> shift) & 255], 1u);
+            const uint64_t act = __ballot(match);
+            if (!act) continue;  // wave-uniform
+            const int lead = __builtin_ctzll(act);
+            const uint32_t d = (uint32_t)(key[j] >> shift) & 255;
+            const uint32_t d0 = __builtin_amdgcn_readlane(d, lead);
+            const uint64_t same = __ballot(match && d == d0);
+            if (lane == lead) atomicAdd(&hist[r][d0], (uint32_t)__popcll(same));
+            else if (match && d != d0) atomicAdd(&hist[r][d], 1u);
         }
         __syncthreads();
-        if (t < 64) {  // one wave scans the 256 bins, 4 per lane
-            const uint32_t h0 = hist[4 * t], h1 = hist[4 * t + 1], h2 = hist[4 * t + 2], h3 = hist[4 * t + 3];
-            const uint32_t tot = h0 + h1 + h2 + h3;
-            uint32_t incl = tot;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t o = __shfl_up(incl, off, DQ_WAVE);
-                if (t >= off) incl += o;
-            }
-            const uint32_t excl = incl - tot;
-            if (excl < rank && rank <= incl) {  // exactly one lane
-                uint32_t c = excl, d = 4 * t;
-                const uint32_t hv[4] = {h0, h1, h2, h3};
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (c + hv[q] >= rank) {
-                        d = 4 * t + q;
-                        break;
-                    }
-                    c += hv[q];
-                }
-                s_prefix = (prefix << 8) | d;
-                s_rank = rank - c;
-                s_bin = hist[d];
-            }
-        }
-        __syncthreads();
-        prefix = s_prefix;
-        rank = s_rank;
-        if (s_bin == 1) {  // one key has this prefix: it is K (uniform branch)
-#pragma unroll
-            for (int j = 0; j < TK_PER; ++j)
-                if ((key[j] >> shift) == prefix) s_key = key[j];
-            __syncthreads();
-            prefix = s_key;
-            break;
-        }
+        // every wave scans the 256 bins, 4 per lane: the bin of the rank-th key
+        const dq_u32x4 h = *reinterpret_cast<const dq_u32x4*>(&hist[r][4 * lane]);
+        const uint32_t incl = wave_scan(h.x + h.y + h.z + h.w);
+        const uint64_t at = __ballot(incl >= rank);  // incl ascends: the first such lane holds the bin
+        const int L = __builtin_ctzll(at);
+        uint32_t below = incl - h.x - h.y - h.z - h.w, d = 4 * lane, cnt = h.x;
+        if (below + cnt < rank) below += cnt, cnt = h.y, ++d;
+        if (below + cnt < rank) below += cnt, cnt = h.z, ++d;
+        if (below + cnt < rank) below += cnt, cnt = h.w, ++d;
+        prefix = (prefix << 8) | __builtin_amdgcn_readlane(d, L);
+        rank -= __builtin_amdgcn_readlane(below, L);
+        whole = rank == __builtin_amdgcn_readlane(cnt, L);
+        if (whole || r == 7) break;  // the same in every wave
     }
-    // prefix is now K, the want-th smallest key. Real keys are distinct, so
-    // exactly `want` keys are <= K - unless K is the padding key ~0 (a later
-    // pass over a chunk holding fewer than kk real keys): then only the keys
-    // below it are taken and the rest of the output is padding again.
-    if (t == 0) s_cnt = 0;
-    __syncthreads();
-    const bool real = prefix != ~0ull;
+    // Real keys are distinct, so a bin of the last round is whole unless it is
+    // that of the padding key ~0 (a later pass over a chunk holding fewer than
+    // kk real keys): then only the keys below it are taken and the rest of the
+    // output is padding again.
+    uint64_t take[TK_PER];
+    uint32_t n_take = 0;
 #pragma unroll
     for (int j = 0; j < TK_PER; ++j) {
-        if (key[j] < prefix || (real && key[j] == prefix)) {
-            const uint32_t pos = atomicAdd(&s_cnt, 1u);
-            if (pos < 256) list[pos] = key[j];
-        }
+        const uint64_t k = key[j] >> shift;
+        take[j] = __ballot(k < prefix || (whole && k == prefix));
+        n_take += __popcll(take[j]);
+    }
+    uint32_t pos = 0;
+    if (n_take) {
+        if (lane == 0) pos = atomicAdd(&s_cnt, n_take);
+        pos = __builtin_amdgcn_readfirstlane(pos);
+    }
+#pragma unroll
+    for (int j = 0; j < TK_PER; ++j) {
+        const uint32_t p = pos + __popcll(take[j] & ((1ull << lane) - 1));
+        if ((take[j] >> lane & 1) && p < 256) list[p] = key[j];
+        pos += __popcll(take[j]);
     }
     __syncthreads();
-    const uint32_t got = s_cnt < want ? s_cnt : want;
-    int P = 1;
-    while (P < (int)kk) P <<= 1;
-    for (int j = got + t; j < P; j += TK_T) list[j] = ~0ull;
-    __syncthreads();
-    if (sorted) {  // the final pass: ids and values, best first
-        bitonic_sort(list, P);
-        for (uint32_t j = t; j < kk; j += TK_T) {
-            if (ids) ids[j] = (int32_t)(uint32_t)list[j];
-            if (vals) vals[j] = key_value(list[j]);
-        }
+    if (!sorted) {
+        for (uint32_t j = t; j < kk; j += TK_S) kout[(size_t)blockIdx.x * kk + j] = list[j];
         return;
     }
-    for (uint32_t j = t; j < kk; j += TK_T) kout[(size_t)blockIdx.x * kk + j] = list[j];
+    // the final pass: ids and values, best first. A key's place is the number
+    // of keys below it (equal ones, padding only, by position), counted by
+    // TK_S / P threads per key.
+    int P = 1;
+    while (P < (int)kk) P <<= 1;
+    const uint32_t i = t & (P - 1);
+    if (i < kk) {
+        const uint64_t own = list[i];
+        uint32_t c = 0;
+        for (uint32_t j = t / P; j < kk; j += TK_S / P) {
+            const uint64_t o = list[j];
+            c += o < own || (o == own && j < i);
+        }
+        if (c) atomicAdd(&order[i], c);
+    }
+    __syncthreads();
+    if (t < (int)kk) {
+        const uint64_t own = list[t];
+        const uint32_t p = order[t];
+        if (ids) ids[p] = (int32_t)(uint32_t)own;
+        if (vals) vals[p] = key_value(own);
+    }
 }
 
 // kk = 1: the smallest key of each chunk.
@@ -399,7 +409,7 @@ int dq_topk(const float* d_v, uint32_t n, uint32_t kk, int32_t* d_ids, float* d_
         const unsigned blocks = (unsigned)((m + TK_CHUNK - 1) / TK_CHUNK);
         const int final = blocks == 1;
         if (kk == 1) argmin_pass_kernel<<<blocks, TK_T, 0, s>>>(d_v, kin, (uint32_t)m, final, buf[cur], d_ids, d_vals);
-        else topk_pass_kernel<<<blocks, TK_T, 0, s>>>(d_v, kin, (uint32_t)m, kk, final, buf[cur], d_ids, d_vals);
+        else topk_pass_kernel<<<blocks, TK_S, 0, s>>>(d_v, kin, (uint32_t)m, kk, final, buf[cur], d_ids, d_vals);
         kin = buf[cur];
         m = (size_t)blocks * kk;
         cur ^= 1;

@@ -39,6 +39,21 @@ def test_topk_exact(gpu, n, kk):
     assert np.array_equal(vals.cpu().numpy(), v[want])
 
 
+@pytest.mark.parametrize("kind", ["equal", "one_binade", "descending", "minus_inf"])
+@pytest.mark.parametrize("n,kk", [(2, 2), (65, 64), (256, 256), (4095, 255), (4100, 104), (12289, 129), (70001, 256)])
+def test_topk_shared_digits(gpu, n, kk, kind):
+    """Keys that share all value digits, or all but the last ones; a last chunk of fewer keys than asked for; as
+    many keys as asked for. Exact."""
+    print(f"topk {kind} n={n} kk={kk}", flush=True)
+    v = {"equal": np.full(n, -3.25), "one_binade": 1 + np.random.default_rng(n).permutation(n) * 2.0 ** -20,
+         "descending": -np.arange(n) / 7, "minus_inf": np.where(np.arange(n) % 97 == 5, 1.5, -np.inf)}[kind]
+    v = v.astype(np.float32)
+    ids, vals = ops.topk(torch.from_numpy(v).to(gpu), kk)
+    want = so.top_k_select(v, kk)
+    assert np.array_equal(ids.cpu().numpy(), want.astype(np.int32))
+    assert np.array_equal(vals.cpu().numpy(), v[want])
+
+
 def sample_args(kk, temperature, top_k, top_p, repeat, freq, present, last_n, u, append=0, slot=0):
     a = _lib.CudaSampleArgs()
     a.temperature, a.top_k, a.top_p = temperature, top_k, top_p
