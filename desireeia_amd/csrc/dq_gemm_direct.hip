@@ -1,4 +1,4 @@
-// dq_gemm_direct.hip - the prefill GEMM for few tokens (up to a few hundred):
+// dq_gemm_direct.hip - the prefill GEMM for few tokens (up to 128):
 // Y[t][r] = sum_k W[r][k] X[t][k], the semantics and operands of dq_gemm.hip
 // (fp16(q_x * dx * s) against fp16(a * q_w), the Q4_K min term as one more
 // MFMA slice per super-block, fp32 accumulation, 1/s on the output).
