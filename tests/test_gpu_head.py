@@ -40,7 +40,7 @@ def test_topk_exact(gpu, n, kk):
 
 
 @pytest.mark.parametrize("kind", ["equal", "one_binade", "descending", "minus_inf"])
-@pytest.mark.parametrize("n,kk", [(2, 2), (65, 64), (256, 256), (4095, 255), (4100, 104), (12289, 129), (70001, 256)])
+@pytest.mark.parametrize("n,kk", [(2, 2), (65, 64), (256, 256), (4095, 255), (4100, 104), (12289, 129), (65537, 256), (70001, 256)])
 def test_topk_shared_digits(gpu, n, kk, kind):
     """Keys that share all value digits, or all but the last ones; a last chunk of fewer keys than asked for; as
     many keys as asked for. Exact."""
